@@ -22,6 +22,8 @@ D3D_INPUT_PROBS = 1
 D3D_ACCEPT_NOALLOC_SCRATCH_BYTES = 4 << 20
 D3D_CONF_MAX_SOFTMAX = 0
 D3D_CONF_ONE_HOT = 1
+FILTER_MAX_K = 4096  # top_k and vocabulary d3d_filter_rows takes
+FILTER_MAX_V = 1 << 18
 D3D_TOKEN_EMPTY_DISTRIBUTION = -1
 D3D_TOKEN_BAD_DRAFT = -2
 D3D_TOKEN_TIMEOUT = -3
@@ -78,6 +80,8 @@ SIGNATURES = {
     "d3d_sample_rows": (_I, [_P, _I, _I, _I64, _F, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "d3d_softmax_rows": (_I, [_P, _I, _I, _I64, _F, _P, _P, _P, _P, _P, _SZ, _P]),
     "d3d_row_filter": (_I, [_P, _I, _I, _I64, _F, _I, _F, _P, _P, _P]),
+    "d3d_filter_rows_workspace_bytes": (_SZ, [_I, _I64]),
+    "d3d_filter_rows": (_I, [_P, _I, _I, _I64, _F, _I, _F, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "d3d_support_workspace_bytes": (_SZ, [_I, _I]),
     "d3d_sample_support_wide": (_I, [_P, _I, _I, _I64, _F, _I, _F, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "d3d_sample_support": (_I, [_P, _P, _I, _I, _F, _F, _P, _P, _P, _P, _P]),

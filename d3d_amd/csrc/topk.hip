@@ -24,11 +24,19 @@
 // zero), so a round is 16 integer maxes, an unsigned-max butterfly and one
 // barrier: 161.8 -> 136.3 us at that shape against the (value, index)
 // compares with a taken mask and two-barrier argmax that fp32 rows keep.
+// The rounds cost k; above 8 (bf16) or 4 (fp32) the group-maxima selection of
+// select.hip is faster.  Rounds / selection, 151,936 entries, 64 rows: bf16
+// k = 4 18.3 / 26.0 us, k = 8 27.9 / 26.2, k = 64 236 / 22; fp32 k = 2 18.5 /
+// 24.8, k = 4 30.7 / 27.1, k = 8 56.1 / 26.8; at 1,088 bf16 rows k = 4 161 /
+// 176, k = 8 235 / 176; one bf16 row k = 8 16.0 / 20.5.
 #include "d3d_common.hpp"
 #include "rowstats.hpp"
+#include "select.hpp"
 #include "../../include/d3d_hip.h"
 
 #include <limits.h>
+
+#include <algorithm>
 
 namespace d3d {
 namespace topk {
@@ -42,6 +50,12 @@ constexpr int kMaxK = 64;
 constexpr int kBf16Chunks = 1;
 template <int DT>
 constexpr int chunks_per_wg() { return DT == kBF16 ? kBf16Chunks : 1; }
+// Largest k taken by rounds; wider ones (and V <= 2^18) go to select.hip.
+#ifdef D3D_TOPK_ROUNDS
+constexpr int rounds_max_k(int) { return D3D_TOPK_ROUNDS; }
+#else
+constexpr int rounds_max_k(int dtype) { return dtype == kF32 ? 4 : 8; }
+#endif
 constexpr int kMaxCand = 8192;  // chunk candidates per row merged in LDS
 
 struct Cand {
@@ -546,10 +560,17 @@ static size_t cand_bytes(int N, int64_t V, int k) {
     return ((size_t)N * C * k * sizeof(topk::Cand) + 255) & ~(size_t)255;
 }
 
+static bool topk_selects(int dtype, int64_t V, int k) { return k > topk::rounds_max_k(dtype) && V <= filt::kMaxV; }
+
 extern "C" size_t d3d_topk_workspace_bytes(int N, int64_t V, int k) {
     if (N < 1 || V < 1 || k < 1) return 0;
     const size_t C = (size_t)((V + rows::kChunk - 1) / rows::kChunk);
-    return cand_bytes(N, V, k) + (((size_t)N * C * sizeof(float2) + 255) & ~(size_t)255);
+    // The dtype is not known here: room for whichever way it takes.
+    size_t bytes = 0;
+    if (topk_selects(D3D_DTYPE_F32, V, k)) bytes = filt::select_scratch_bytes(N, (int)C, true);
+    if (!topk_selects(D3D_DTYPE_BF16, V, k))
+        bytes = std::max(bytes, cand_bytes(N, V, k) + (((size_t)N * C * sizeof(float2) + 255) & ~(size_t)255));
+    return bytes;
 }
 
 extern "C" int d3d_topk_rows(const void* logits, int dtype, int N, int64_t V, int k, int log_softmax,
@@ -570,6 +591,9 @@ extern "C" int d3d_topk_rows(const void* logits, int dtype, int N, int64_t V, in
     P.k = k;
     if ((int64_t)P.C * k > kMaxCand) return D3D_E_SHAPE;
     if (workspace_bytes < d3d_topk_workspace_bytes(N, V, k)) return D3D_E_WORKSPACE;
+    if (topk_selects(dtype, V, k))
+        return (int)filt::select_topk(logits, dtype, N, (int)V, k, log_softmax && vals_out, ids_out, vals_out,
+                                      workspace, static_cast<hipStream_t>(stream));
     P.cand = static_cast<Cand*>(workspace);
     P.lse = (log_softmax && vals_out)
                 ? reinterpret_cast<float2*>(static_cast<char*>(workspace) + cand_bytes(N, V, k))

@@ -111,32 +111,41 @@ def _uniforms(shape, dev, uniforms, generator):
     return uniforms.to(device=dev, dtype=torch.float32).reshape(shape).contiguous()
 
 
-def _filters(logits: torch.Tensor, temperature: float, top_k: int, top_p: Optional[float]):
-    """The top-k / top-p filter of _sampling_probs (single/eval_sync.py:
-    292-303) for rows [N, V]: (kth, None, None) with kth the per-row k-th
-    largest logit for a top-k filter alone of at most 64 entries (one top-k
-    launch pair), (None, zfloor, zlimit) from d3d_row_filter for top-p or a
-    wider top-k, (None, None, None) when both are off."""
-    V = logits.shape[-1]
+def _filter_args(V: int, top_k: int, top_p: Optional[float]) -> Tuple[int, float, bool]:
+    """(k, p, fused): the top-k (0: off) and top-p (1: off) filters of
+    _sampling_probs (single/eval_sync.py:292-303) for rows of V entries, and
+    whether d3d_filter_rows takes them (it needs a filter)."""
     k = int(top_k) if top_k and top_k > 0 else 0
     if k >= V:
         k = 0
     p = 1.0 if top_p is None else float(top_p)
     if not 0.0 < p <= 1.0:
         raise ValueError("top_p must lie in (0, 1]")
+    return k, p, (k > 0 or p < 1.0) and k <= _lib.FILTER_MAX_K and V <= _lib.FILTER_MAX_V
+
+
+def _filters(logits: torch.Tensor, temperature: float, k: int, p: float, fused: bool):
+    """The filter of _filter_args for rows [N, V] as (zfloor, zlimit), (None,
+    None) when it is off."""
     if p >= 1.0 and k == 0:
-        return None, None, None
-    if p >= 1.0 and k <= 64:
-        _, vals = topk_tokens(logits, k, with_values=True)
-        return vals[..., k - 1].reshape(-1).contiguous(), None, None
+        return None, None
+    V = logits.shape[-1]
     N = logits.numel() // V
     dev = logits.device
     zf = torch.empty(N, dtype=torch.float32, device=dev)
     lim = torch.empty(N, dtype=torch.int32, device=dev)
-    st = _lib.load().d3d_row_filter(logits.data_ptr(), _lib.dtype_code(logits), N, V, float(temperature), k, p,
-                                    zf.data_ptr(), lim.data_ptr(), _lib.stream_ptr(dev))
-    _lib.check(st, "d3d_row_filter")
-    return None, zf, lim
+    lib = _lib.load()
+    if fused:
+        ws = _lib.workspace(dev, "filter", lib.d3d_filter_rows_workspace_bytes(max(N, 1), V))
+        st = lib.d3d_filter_rows(logits.data_ptr(), _lib.dtype_code(logits), N, V, float(temperature), k, p, None,
+                                 zf.data_ptr(), lim.data_ptr(), None, None, ws.data_ptr(), ws.numel(),
+                                 _lib.stream_ptr(dev))
+        _lib.check(st, "d3d_filter_rows")
+    else:
+        st = lib.d3d_row_filter(logits.data_ptr(), _lib.dtype_code(logits), N, V, float(temperature), k, p,
+                                zf.data_ptr(), lim.data_ptr(), _lib.stream_ptr(dev))
+        _lib.check(st, "d3d_row_filter")
+    return zf, lim
 
 
 def sample_with_prob(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 0, top_p: float = 1.0, *,
@@ -157,12 +166,20 @@ def sample_with_prob(logits: torch.Tensor, temperature: float = 0.0, top_k: int 
     N = lg.numel() // V
     greedy = not temperature > 1e-5
     u = None if greedy else _uniforms(lg.shape[:-1], dev, uniforms, generator)
-    kth, zf, lim = (None, None, None) if greedy else _filters(lg, temperature, top_k, top_p)
+    k, p, fused = (0, 1.0, False) if greedy else _filter_args(V, top_k, top_p)
     tok = torch.empty(lg.shape[:-1], dtype=torch.int64, device=dev)
     prob = torch.empty(lg.shape[:-1], dtype=torch.float32, device=dev)
     lib = _lib.load()
+    if fused:
+        ws = _lib.workspace(dev, "filter", lib.d3d_filter_rows_workspace_bytes(max(N, 1), V))
+        st = lib.d3d_filter_rows(lg.data_ptr(), _lib.dtype_code(lg), N, V, float(temperature), k, p, u.data_ptr(),
+                                 None, None, tok.data_ptr(), prob.data_ptr(), ws.data_ptr(), ws.numel(),
+                                 _lib.stream_ptr(dev))
+        _lib.check(st, "d3d_filter_rows")
+        return tok, prob
+    zf, lim = _filters(lg, temperature, k, p, fused)
     ws = _lib.workspace(dev, "sample", lib.d3d_sample_workspace_bytes(max(N, 1), V))
-    st = lib.d3d_sample_rows(lg.data_ptr(), _lib.dtype_code(lg), N, V, float(temperature), _lib.ptr(kth),
+    st = lib.d3d_sample_rows(lg.data_ptr(), _lib.dtype_code(lg), N, V, float(temperature), None,
                              _lib.ptr(zf), _lib.ptr(lim), _lib.ptr(u), tok.data_ptr(), prob.data_ptr(),
                              ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
     _lib.check(st, "d3d_sample_rows")
@@ -191,11 +208,11 @@ def sampling_probs(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 
     V = lg.shape[-1]
     N = lg.numel() // V
     greedy = not temperature > 1e-5
-    kth, zf, lim = (None, None, None) if greedy else _filters(lg, temperature, top_k, top_p)
+    zf, lim = (None, None) if greedy else _filters(lg, temperature, *_filter_args(V, top_k, top_p))
     out = torch.empty(lg.shape, dtype=torch.float32, device=dev)
     lib = _lib.load()
     ws = _lib.workspace(dev, "sample", lib.d3d_sample_workspace_bytes(max(N, 1), V))
-    st = lib.d3d_softmax_rows(lg.data_ptr(), _lib.dtype_code(lg), N, V, float(temperature), _lib.ptr(kth),
+    st = lib.d3d_softmax_rows(lg.data_ptr(), _lib.dtype_code(lg), N, V, float(temperature), None,
                               _lib.ptr(zf), _lib.ptr(lim), out.data_ptr(), ws.data_ptr(), ws.numel(),
                               _lib.stream_ptr(dev))
     _lib.check(st, "d3d_softmax_rows")
@@ -212,8 +229,8 @@ def sample_with_sparse_probs(logits: torch.Tensor, temperature: float, top_k: in
     probabilities are softmax(z) over the support after the nucleus filter
     (``top_p`` < 1: entry s > 0 is dropped when the mass of entries 0..s-1
     exceeds top_p), and the token is the inverse-CDF draw from them in
-    support order.  Supports of up to 64 entries take the top-k kernel and
-    one wave per row; wider ones the sorted-support path.
+    support order.  Supports of up to 8 entries take the top-k rounds and one
+    wave per row; wider ones the sorted-support path.
     """
     dev = _lib.require_device(logits)
     if not temperature > 1e-5:
@@ -231,7 +248,7 @@ def sample_with_sparse_probs(logits: torch.Tensor, temperature: float, top_k: in
     u = _uniforms(lg.shape[:-1], dev, uniforms, generator)
     tok = torch.empty(lg.shape[:-1], dtype=torch.int64, device=dev)
     probs = torch.empty(*lg.shape[:-1], S, dtype=torch.float32, device=dev)
-    if S > 64:
+    if S > 8:
         ids = torch.empty(*lg.shape[:-1], S, dtype=torch.int64, device=dev)
         lib = _lib.load()
         nbytes = lib.d3d_support_workspace_bytes(max(N, 1), S)

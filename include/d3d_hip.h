@@ -400,6 +400,27 @@ int d3d_softmax_rows(const void* logits, int dtype, int N, int64_t V, float temp
 int d3d_row_filter(const void* logits, int dtype, int N, int64_t V, float temperature, int top_k, float top_p,
                    float* zfloor_out, int32_t* zlimit_out, void* stream);
 
+/* Bytes of workspace d3d_filter_rows needs (bounded: rows are taken in
+ * batches of 256); 0 for V > 2^18. */
+size_t d3d_filter_rows_workspace_bytes(int N, int64_t V);
+
+/*
+ * d3d_row_filter and, with tokens_out, the draw of d3d_sample_rows under that
+ * filter, for V <= 2^18 and top_k <= 4096 (0 or >= V: off, then top_p < 1):
+ * two launches with a top-k, four without, instead of several passes by one
+ * workgroup per row.  zfloor_out / zlimit_out [N] (both or neither), as
+ * d3d_row_filter; tokens_out [N] (needs uniforms [N]) and probs_out [N] (may
+ * be NULL): the inverse-CDF draw over the kept entries in id order and its
+ * probability.  Masses are sums of exp(z - max z) in 2^-40 units.  Larger
+ * top_k: D3D_E_UNSUPPORTED (d3d_row_filter takes any).
+ *
+ * Replaces _sampling_probs' filters and _sample_with_prob,
+ * single/eval_sync.py:287-338.
+ */
+int d3d_filter_rows(const void* logits, int dtype, int N, int64_t V, float temperature, int top_k, float top_p,
+                    const float* uniforms, float* zfloor_out, int32_t* zlimit_out, int64_t* tokens_out,
+                    float* probs_out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Bytes of workspace d3d_sample_support_wide needs. */
 size_t d3d_support_workspace_bytes(int N, int S);
 
@@ -413,8 +434,9 @@ size_t d3d_support_workspace_bytes(int N, int S);
  * renormalised), tokens_out [N] = the inverse-CDF draw over the support in
  * support order at uniforms[n], token_probs_out [N] (may be NULL) its
  * probability.  T > 1e-5, 0 < top_p <= 1.  Workspace:
- * d3d_support_workspace_bytes(N, S).  d3d_topk_rows + d3d_sample_support
- * cover S <= 64 in one launch pair.
+ * d3d_support_workspace_bytes(N, S).  Two launches for S <= 4096 (a
+ * selection in LDS), a segmented sort above.  d3d_topk_rows +
+ * d3d_sample_support cover S <= 64 too and are faster up to 8.
  */
 int d3d_sample_support_wide(const void* logits, int dtype, int N, int64_t V, float temperature, int S,
                             float top_p, const float* uniforms, int64_t* tokens_out, int64_t* support_ids_out,

@@ -1,0 +1,141 @@
+"""The candidate-based top-k and nucleus kernels (GPU) at their edges.
+
+d3d_filter_rows must give the filter of d3d_row_filter (the general
+multi-pass selection) bit for bit: both place the cut with the same exact
+64-bit masses.  Its draw is checked against the draw of d3d_sample_rows under
+that filter, whose fp32 masses may cross a bar edge the other way.  Supports
+and top-k are checked against a stable CPU sort.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from d3d_amd import _lib
+from d3d_amd import draft as dr
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+INF = float("inf")
+
+
+def _rows(kind, N, V, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(N, V, generator=g) * 2.0
+    if kind == "ties":       # few distinct values: long runs at every cut
+        x = x.round()
+    elif kind == "flat":     # one value per row: no candidate list holds it
+        x = torch.zeros(N, V)
+        x[:, V // 2] = 1.0
+    elif kind == "masked":   # most of the vocabulary at -inf
+        x[:, ::2] = -INF
+        x[N // 2:, 40:] = -INF
+    elif kind == "odd":      # NaN, infinities, zeros, denormals, a far outlier
+        x[0, ::7] = float("nan")
+        x[1, 5] = INF
+        x[2, :] = -INF
+        x[3, ::3] = 0.0
+        x[3, 1::3] = 1e-41
+        x[4, V - 1] = 3e38
+    elif kind == "sorted":   # the k largest are neighbours: few groups hold them
+        x = x.sort(-1, descending=True).values
+    return x.to(dtype).to(DEV)
+
+
+def _general(x, T, k, p):
+    N, V = x.shape
+    zf = torch.empty(N, device=DEV)
+    lim = torch.empty(N, dtype=torch.int32, device=DEV)
+    st = _lib.load().d3d_row_filter(x.data_ptr(), _lib.dtype_code(x), N, V, T, k, p, zf.data_ptr(), lim.data_ptr(),
+                                    _lib.stream_ptr(DEV))
+    _lib.check(st, "d3d_row_filter")
+    return zf, lim
+
+
+def _draw(x, T, zf, lim, u):
+    N, V = x.shape
+    tok = torch.empty(N, dtype=torch.int64, device=DEV)
+    prob = torch.empty(N, device=DEV)
+    lib = _lib.load()
+    ws = torch.empty(lib.d3d_sample_workspace_bytes(N, V), dtype=torch.uint8, device=DEV)
+    st = lib.d3d_sample_rows(x.data_ptr(), _lib.dtype_code(x), N, V, T, None, zf.data_ptr(), lim.data_ptr(),
+                             u.data_ptr(), tok.data_ptr(), prob.data_ptr(), ws.data_ptr(), ws.numel(),
+                             _lib.stream_ptr(DEV))
+    _lib.check(st, "d3d_sample_rows")
+    return tok, prob
+
+
+@pytest.mark.parametrize("kind", ["plain", "ties", "flat", "masked", "odd", "sorted"])
+@pytest.mark.parametrize("V,k,p", [(151936, 0, 0.9), (151936, 0, 0.05), (32771, 0, 0.999), (4097, 0, 0.5),
+                                   (151936, 1, 1.0), (151936, 64, 0.8), (32771, 257, 0.3), (151936, 1025, 1.0),
+                                   (8192, 4096, 0.9), (20000, 300, 1.0), (9, 4, 0.6), (262144, 2000, 0.95)])
+@pytest.mark.parametrize("dtype,T", [(torch.bfloat16, 0.7), (torch.float32, 1.3), (torch.float32, 1.0)])
+def test_filter_rows_equals_the_general_filter(kind, V, k, p, dtype, T):
+    N = 6
+    x = _rows(kind, N, V, dtype, V + k)
+    u = torch.rand(N, generator=torch.Generator().manual_seed(k)).to(DEV)
+    zf, lim = _general(x, T, k, p)
+    kk, pp, fused = dr._filter_args(V, k, p)
+    assert fused
+    got = dr._filters(x, T, kk, pp, fused)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], zf) and torch.equal(got[1], lim)
+    tok, prob = dr.sample_with_prob(x, T, k, p, uniforms=u)
+    rt, rp = _draw(x, T, zf, lim, u)
+    same = tok == rt
+    # The fp32 sums are good to ~1e-6 of the row's mass; only a draw that close
+    # to a bar edge (bars are ~1e-5 wide) may take the neighbour.
+    assert same.float().mean() >= 0.6
+    rows = torch.nonzero(same)[:, 0]
+    # blocked fp32 sums of positive terms: under 2^7 roundings of 2^-24 each side
+    assert torch.allclose(prob[rows], rp[rows], rtol=2e-5, atol=1e-9)
+    # The other rows drew a kept entry too.
+    for n in torch.nonzero(~same)[:, 0].tolist():
+        z = x[n].float() / T
+        t = int(tok[n])
+        assert t >= 0 and (z[t] > zf[n] or (z[t] == zf[n] and t <= lim[n]))
+
+
+def test_filter_rows_takes_rows_in_batches():
+    """More rows than one batch (256), whose scratch the next batch reuses."""
+    N, V = 520, 6001
+    x = _rows("plain", N, V, torch.bfloat16, 4)
+    u = torch.rand(N, device=DEV)
+    for k, p in ((0, 0.9), (70, 0.9)):
+        zf, lim = _general(x, 0.8, k, p)
+        got = dr._filters(x, 0.8, k, p, True)
+        tok, _ = dr.sample_with_prob(x, 0.8, k, p, uniforms=u)
+        one, _ = dr.sample_with_prob(x[300:301], 0.8, k, p, uniforms=u[300:301])
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], zf) and torch.equal(got[1], lim) and torch.equal(tok[300:301], one)
+
+
+def _sorted_ids(x, T, S):
+    z = (x.float().cpu() / T).numpy().astype(np.float32)
+    out = np.full((z.shape[0], S), -1, np.int64)
+    for n, row in enumerate(z):
+        row = np.where(row == 0, np.float32(0), row)
+        key = np.where(np.isnan(row), -np.inf, row)
+        order = np.lexsort((np.arange(row.size), np.isnan(row), -key))
+        out[n] = order[:S]
+    return out
+
+
+@pytest.mark.parametrize("kind", ["plain", "ties", "flat", "masked", "sorted"])
+@pytest.mark.parametrize("V,S", [(151936, 9), (151936, 64), (32771, 256), (32771, 512), (20000, 513), (9000, 4096),
+                                 (16, 9), (12, 12)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_support_and_topk_match_a_stable_sort(kind, V, S, dtype):
+    N, T = 3, 0.8
+    x = _rows(kind, N, V, dtype, V + S)
+    u = torch.rand(N, generator=torch.Generator().manual_seed(S)).to(DEV)
+    tok, ids, probs = dr.sample_with_sparse_probs(x, T, S, 0.95, uniforms=u)
+    ref = _sorted_ids(x, T, S)
+    np.testing.assert_array_equal(ids.cpu().numpy(), ref)
+    assert torch.allclose(probs.sum(-1), torch.ones(N, device=DEV), rtol=1e-5)
+    assert bool((ids == tok[:, None]).any(-1).all())
+    if S <= 64:
+        top, vals = dr.topk_tokens(x, S, with_values=True)
+        np.testing.assert_array_equal(top.cpu().numpy(), _sorted_ids(x, 1.0, S))
+        assert torch.equal(vals, x.float().gather(1, top))
