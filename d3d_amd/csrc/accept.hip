@@ -308,30 +308,7 @@ __device__ __forceinline__ Decision decide(const Params& P, int b, bool writer) 
 // Entries e0 .. e0 + kRun - 1 of a row (fill past V).
 template <int DT, bool VEC, Mode M>
 __device__ __forceinline__ void load_run(const void* row, int V, int e0, float (&x)[kRun]) {
-    constexpr int E = Vec<DT>::E;
-    if (VEC && e0 + kRun <= V) {
-#pragma unroll
-        for (int j = 0; j < kRun / E; ++j) {
-            if constexpr (DT == kF32) {
-                const f32x4 v = reinterpret_cast<const f32x4*>(static_cast<const float*>(row) + e0)[j];
-                x[j * 4 + 0] = v.x;
-                x[j * 4 + 1] = v.y;
-                x[j * 4 + 2] = v.z;
-                x[j * 4 + 3] = v.w;
-            } else {
-                const u32x4 v = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(row) + e0)[j];
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    x[j * 8 + 2 * h] = bf16_bits_to_f32(w[h] & 0xffffu);
-                    x[j * 8 + 2 * h + 1] = bf16_bits_to_f32(w[h] >> 16);
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) x[k] = e0 + k < V ? load_one<DT>(row, e0 + k) : fill_value<M>();
-    }
+    load_tile<DT, VEC, false, kRun>(row, V, e0, Vec<DT>::E, fill_value<M>(), x);
 }
 
 // Weights of this thread's run of part q: wr = the residual max(p - q, 0)

@@ -55,77 +55,74 @@ __device__ __forceinline__ float load_one(const void* row, int e) {
     }
 }
 
-// Loads L entries of one row into x[]: x[j*E + k] holds entry
-// first + j*stride + k.  Entries at or beyond V read as FILL (-inf for logits,
-// 0 for probabilities), which leaves every reduction unchanged, so the
-// arithmetic loops carry no bounds checks.  STREAM marks a single-use read
-// (non-temporal hint).
-template <int DT, bool VEC, bool STREAM, int LT>
-__device__ __forceinline__ void load_tile(const void* row, int V, int first, int stride, float fill,
-                                          float (&x)[LT]) {
-    constexpr int E = Vec<DT>::E;
+// 16 bytes of a row at any element alignment (gfx950 global loads need no
+// more in the unaligned access mode the HSA ABI runs in).
+typedef uint32_t u32x4_el __attribute__((ext_vector_type(4), aligned(2)));
+
+template <bool VEC, bool STREAM>
+__device__ __forceinline__ u32x4 load16(const void* p) {
+    if constexpr (VEC) {
+        const u32x4* q = static_cast<const u32x4*>(p);
+        return STREAM ? __builtin_nontemporal_load(q) : *q;
+    } else {
+        const u32x4_el* q = static_cast<const u32x4_el*>(p);
+        return STREAM ? __builtin_nontemporal_load(q) : *q;
+    }
+}
+
+template <int DT>
+__device__ __forceinline__ void unpack16(u32x4 v, float* x) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int j = 0; j < LT / E; ++j) {
-        const int e0 = first + j * stride;
-        if (VEC && e0 + E <= V) {
-            if constexpr (DT == kF32) {
-                const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(row) + e0);
-                const f32x4 v = STREAM ? __builtin_nontemporal_load(p) : *p;
-                x[j * E + 0] = v.x;
-                x[j * E + 1] = v.y;
-                x[j * E + 2] = v.z;
-                x[j * E + 3] = v.w;
-            } else {
-                const u32x4* p = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(row) + e0);
-                const u32x4 v = STREAM ? __builtin_nontemporal_load(p) : *p;
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    x[j * E + 2 * h] = bf16_bits_to_f32(w[h] & 0xffffu);
-                    x[j * E + 2 * h + 1] = bf16_bits_to_f32(w[h] >> 16);
-                }
-            }
+    for (int h = 0; h < 4; ++h) {
+        if constexpr (DT == kF32) {
+            x[h] = __uint_as_float(w[h]);
         } else {
-#pragma unroll
-            for (int k = 0; k < E; ++k) {
-                const int e = e0 + k;
-                x[j * E + k] = e < V ? load_one<DT>(row, e) : fill;
-            }
+            x[2 * h] = bf16_bits_to_f32(w[h] & 0xffffu);
+            x[2 * h + 1] = __uint_as_float(w[h] & 0xffff0000u);
         }
     }
 }
 
-// As load_tile, for the first nv (runtime, <= LT/E) vectors only.
-template <int DT, bool VEC, int LT>
-__device__ __forceinline__ void load_tile_n(const void* row, int V, int first, int stride, int nv, float fill,
-                                            float (&x)[LT]) {
+// Loads LT entries of one row into x[]: x[j*E + k] holds entry
+// first + j*stride + k.  Entries at or beyond V read as FILL (-inf for logits,
+// 0 for probabilities), which leaves every reduction unchanged, so the
+// arithmetic loops carry no bounds checks.  STREAM marks a single-use read
+// (non-temporal hint).  VEC: the row is 16-byte aligned and V a multiple of
+// E, so a vector lies wholly inside the row or past it.
+//
+// Every vector is loaded before any is unpacked, from an address clamped into
+// the row: with a bounds branch per vector the compiler waited for each load
+// inside its branch, one 16-byte load in flight per thread.  Rows that are not
+// 16-byte aligned (an odd vocabulary) take the same vector loads at element
+// alignment; only a row's last, partial vector is read entry by entry.  64
+// rows, bf16 / fp32, before and after (scalar loads at 151,935 before):
+//   151,936  top-2 14.5 / 18.1 -> 13.9 / 17.5 us, draw 19.7 / 20.8 -> 18.7 / 20.0
+//   151,935  top-2 20.8 / 19.1 -> 13.6 / 18.1 us, draw 26.7 / 22.4 -> 18.7 / 20.5,
+//            acceptance (4 requests, 124 rows) 39.2 / 35.0 -> 27.7 / 29.2
+template <int DT, bool VEC, bool STREAM, int LT>
+__device__ __forceinline__ void load_tile(const void* row, int V, int first, int stride, float fill, float (&x)[LT]) {
     constexpr int E = Vec<DT>::E;
+    const char* base = static_cast<const char*>(row);
+    const bool wide = VEC || V >= E;
+    u32x4 v[LT / E];
+    if (wide) {
+#pragma unroll
+        for (int j = 0; j < LT / E; ++j)
+            v[j] = load16<VEC, STREAM>(base + (size_t)min(first + j * stride, V - E) * Vec<DT>::bytes);
+    }
 #pragma unroll
     for (int j = 0; j < LT / E; ++j) {
-        if (j >= nv) break;
         const int e0 = first + j * stride;
-        if (VEC && e0 + E <= V) {
-            if constexpr (DT == kF32) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(static_cast<const float*>(row) + e0);
-                x[j * E + 0] = v.x;
-                x[j * E + 1] = v.y;
-                x[j * E + 2] = v.z;
-                x[j * E + 3] = v.w;
-            } else {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(row) + e0);
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        if (wide) {
+            float t[E];
+            unpack16<DT>(v[j], t);
 #pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    x[j * E + 2 * h] = bf16_bits_to_f32(w[h] & 0xffffu);
-                    x[j * E + 2 * h + 1] = bf16_bits_to_f32(w[h] >> 16);
-                }
-            }
-        } else {
+            for (int k = 0; k < E; ++k) x[j * E + k] = e0 + E <= V ? t[k] : fill;
+        }
+        if (!VEC && (!wide || (e0 < V && e0 + E > V))) {
 #pragma unroll
-            for (int k = 0; k < E; ++k) {
-                const int e = e0 + k;
-                x[j * E + k] = e < V ? load_one<DT>(row, e) : fill;
-            }
+            for (int k = 0; k < E; ++k) x[j * E + k] = e0 + k < V ? load_one<DT>(row, e0 + k) : fill;
         }
     }
 }
