@@ -1,31 +1,48 @@
-// Weight-streaming GEMM for blocks of at most 64 rows:  Y[M, N] = X[M, K] W[N, K]^T
-// (bf16 in, fp32 accumulation), the projections of a 64-token verify or draft
-// block (serving/vendor/ssd/layers/linear.py: F.linear on bf16 weights).
+// Weight-streaming GEMM for blocks of at most 192 rows:  Y[M, N] = X[M, K] W[N, K]^T
+// (bf16 in, fp32 accumulation), the projections of a verify or draft block of
+// up to twelve requests (serving/vendor/ssd/layers/linear.py: F.linear on bf16
+// weights).
 //
-// At M <= 64 the weights dominate the traffic (a 64-row block reads each
-// weight once and each activation once per 64 output columns), so the
+// Each weight is read once, each activation once per column tile, so the
 // kernel is built to stream W:
 //
-// * Workgroup (column tile of 64, K split s), four waves; each k step moves
-//   a 64 x 128 tile of W and the 64 x 128 tile of X.  Every wave
-//   instruction reads four full 256-byte row segments (16 bytes per lane),
-//   the order that streams the weights fastest of those measured.  Within
-//   a row the 16-byte chunk q is stored at slot q ^ (row & 7) of LDS, so
-//   the MFMA operand reads of 16 consecutive rows spread over the banks.
-// * Register-staged pipeline (gemm_rows64_kernel): the loads of the next
-//   two k steps are in flight in registers while a step is stored to one of
-//   two LDS buffers and multiplied from it, one barrier per step.  The k
-//   loop is unrolled for the step counts the models use (STEPS), so the
-//   compiler's wait before each store counts exactly the loads issued after
-//   it.  Measured against the earlier form (direct global -> LDS loads, two
-//   stages, two barriers per step; kept as gemm_rows64_dma_kernel for other
-//   step counts), graph-replayed on HBM-resident weights: target o 14.7 ->
-//   9.9 us, target down 29.8 -> 23.5, draft qkv 9.2 -> 7.1, draft o 6.7 ->
-//   6.0, draft down 12.4 -> 8.9; the same kernel without loads of X or
-//   without the MFMAs was only 10-15 % faster, so the direct-to-LDS loads
-//   with one stage ahead were the bound.
-// * Wave w multiplies the 64 rows of X by columns 16w .. 16w + 15 of the
-//   tile with v_mfma_f32_16x16x32_bf16, both operands read from LDS.
+// * Workgroup (column tile of TN, K split s); each k step moves a TN x TK tile
+//   of W and the MR x TK tile of X (MR: M rounded up to 16, 32, 64, 128 or
+//   192).  Every wave instruction reads whole 128- or 256-byte row segments
+//   (16 bytes per lane), the order that streams the weights fastest of those
+//   measured.  Within a row the 16-byte chunk q is stored at slot q ^ (row & 7)
+//   of LDS, so the MFMA operand reads of 16 consecutive rows spread over the
+//   banks.
+// * Register-staged pipeline (rows_kernel): the loads of the next P k steps
+//   are in flight in registers while a step is stored to one of two LDS
+//   buffers and multiplied from it, one barrier per step.  The k loop is
+//   unrolled for the step counts the models use (STEPS), so the compiler's
+//   wait before each store counts exactly the loads issued after it; as a
+//   loop, with a wait for every load at its head, it ran 5-12 % longer.
+//   Other step counts of up to 64 rows run on gemm_rows64_dma_kernel (direct
+//   global -> LDS loads, two stages, two barriers per step).
+// * The tile per row count (us, graph-replayed on HBM-resident weights; the
+//   weights alone take 10.3 / 6.8 / 20.5 us at the copy rate for the target's
+//   qkv / o / down, 3.4 / 1.7 / 5.1 for the draft's):
+//     M <= 16, 32: four waves, TK 128.  In the 64-row kernel three quarters
+//       of the X loads, LDS traffic and MFMAs were repeats of the last row.
+//       16 rows: target 12.9 / 8.3 / 19.7 -> 11.5 / 7.5 / 18.7, draft
+//       5.9 / 4.3 / 7.3 -> 5.0 / 3.8 / 6.3.
+//     M <= 64: four waves, TK 64, three stages in flight: target
+//       15.4 / 10.0 / 22.4 -> 15.6 / 9.6 / 22.6, draft 7.3 / 5.6 / 8.9 ->
+//       6.8 / 5.6 / 8.4 against TK 128 and two stages.
+//     M <= 128, 192: eight waves, TK 64, two stages (hipBLASLt before).
+//       128 rows: target 25.7 / 24.4 / 67.4 -> 19.7 / 12.3 / 29.8, draft
+//       14.7 / 11.2 / 17.8 -> 8.6 / 6.9 / 10.9; 192 rows: target
+//       34.4 / 33.2 / 90.8 -> 24.3 / 15.4 / 37.0, draft 21.4 / 11.9 / 22.6 ->
+//       10.7 / 8.4 / 13.4.  Every workgroup reads the whole X of its k range
+//       through L2, which is what grows with M: four waves with TK 128 took
+//       22.8 / 15.3 / 34.9 at 128 rows (one wave per SIMD, nothing beside its
+//       LDS reads), column tiles of 128 halve that traffic but leave half the
+//       CUs idle at these splits (25.4 / 16.0 / 38.9).
+// * The waves split the tile (WR rows of waves x WC columns) and multiply
+//   with v_mfma_f32_16x16x32_bf16, both operands read from LDS.  The sum over
+//   k of an entry runs in the same order in every variant.
 // * Small N leaves too few column tiles to fill 256 CUs, so K is split over
 //   `splits` workgroups per tile (d3d_gemm_rows64_splits picks the count).
 //   With one split the result is rounded to bf16 into Y; with several,
@@ -34,15 +51,13 @@
 //   d3d_qk_rope_append_parts) -- no extra launch, no atomics, and the sum
 //   has the same bits on every call.
 #include "d3d_common.hpp"
+#include "gemm_rows.hpp"
 #include "../../include/d3d_hip.h"
 
 namespace d3d {
 namespace gemm {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
+// gemm_rows64_dma_kernel's tiles.
 constexpr int NT = 256;                  // four waves
 constexpr int TN = 64;                   // output columns per workgroup
 constexpr int TK = 128;                  // k per stage
@@ -158,95 +173,6 @@ __global__ __launch_bounds__(NT) void gemm_rows64_dma_kernel(const uint16_t* __r
     store_tile(acc, y, parts, M, N, n0 + 16 * wv + c16, g4);
 }
 
-// Register-staged form of the kernel above (same tiles, LDS layout and
-// results): stage st of a lane is rw / rx[st % 2] until it is stored to
-// LDS buffer st % 2; the loads of stage st + 2 then reuse those registers.
-//
-// SILU: W is a gate-up weight [2 H, K] (gate rows, then up rows) and Y
-// [M, H] = silu(bf16(X Wg^T)) * bf16(X Wu^T), each product rounded as the
-// bf16 GEMM output would be, then evaluated as d3d_silu_mul does.  Tile t
-// stands for output columns 32 t .. 32 t + 31: tile row 16 w + c is gate
-// row 32 t + 8 w + c (c < 8) or the up row of column 32 t + 8 w + c - 8, so
-// a lane's gate and up products of one column sit in lanes c and c + 8 of
-// its 16-lane row.
-template <int STEPS, bool SILU = false>
-__global__ __launch_bounds__(NT, 2) void gemm_rows64_kernel(const uint16_t* __restrict__ x,
-                                                            const uint16_t* __restrict__ w,
-                                                            uint16_t* __restrict__ y, float* __restrict__ parts,
-                                                            int M, int N, int K, int KR) {
-    constexpr int P = 2;  // k steps in flight in registers
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    const int c16 = lane & 15, g4 = lane >> 4;
-    const int n0 = blockIdx.x * TN;
-    const int kb = blockIdx.y * KR;
-    // This lane's source rows and LDS slots: wave wv loads rows
-    // (wv * LPW + j) * RPI + lane / CPR of both tiles, global chunk
-    // (lane % CPR) ^ (row & 7) into LDS chunk lane % CPR.
-    const int lr = lane / CPR, lc = lane % CPR;
-    const uint16_t* wsrc[LPW];
-    const uint16_t* xsrc[LPW];
-    int lofs[LPW];
-#pragma unroll
-    for (int j = 0; j < LPW; ++j) {
-        const int r = (wv * LPW + j) * RPI + lr;
-        const int q = lc ^ (r & 7);
-        int wrow = n0 + r;
-        if constexpr (SILU) {
-            const int col = 32 * blockIdx.x + 8 * (r >> 4) + (r & 7);
-            wrow = (r & 8) ? N / 2 + col : col;
-        }
-        wsrc[j] = w + (size_t)wrow * K + kb + 8 * q;
-        xsrc[j] = x + (size_t)min(r, M - 1) * K + kb + 8 * q;
-        lofs[j] = r * ROWB + lc * 16;
-    }
-    u32x4 rw[P][LPW], rx[P][LPW];
-    auto load = [&](int st, int sl) {
-#pragma unroll
-        for (int j = 0; j < LPW; ++j) {
-            rw[sl][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wsrc[j] + st * TK));
-            rx[sl][j] = *reinterpret_cast<const u32x4*>(xsrc[j] + st * TK);
-        }
-    };
-    f32x4 acc[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) acc[t] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int p = 0; p < P; ++p)
-        if (p < STEPS) load(p, p);
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) {
-        // Buffer st % 2 was last read in step st - 2, which every wave
-        // finished before the barrier of step st - 1.
-        char* buf = smem + (st & 1) * STAGEB;
-#pragma unroll
-        for (int j = 0; j < LPW; ++j) {
-            *reinterpret_cast<u32x4*>(buf + lofs[j]) = rw[st % P][j];
-            *reinterpret_cast<u32x4*>(buf + TILEB + lofs[j]) = rx[st % P][j];
-        }
-        if (st + P < STEPS) load(st + P, st % P);
-        __syncthreads();
-        mma_step(buf, acc, wv, c16, g4);
-    }
-    if constexpr (SILU) {
-        const int H = N / 2, col = 32 * blockIdx.x + 8 * wv + (c16 & 7);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float mine = acc[t][r], other = __shfl_xor(mine, 8, kWave);
-                const int m = 16 * t + 4 * g4 + r;
-                if (c16 < 8 && m < M) {
-                    const float gv = bf16_bits_to_f32(f32_to_bf16_bits(mine));
-                    const float uv = bf16_bits_to_f32(f32_to_bf16_bits(other));
-                    y[(size_t)m * H + col] = __builtin_bit_cast(uint16_t, (__bf16)(gv / (1.0f + expf(-gv)) * uv));
-                }
-            }
-    } else {
-        store_tile(acc, y, parts, M, N, n0 + 16 * wv + c16, g4);
-    }
-}
-
 }  // namespace gemm
 }  // namespace d3d
 
@@ -271,55 +197,82 @@ extern "C" int d3d_gemm_rows64_splits(int N, int K) {
     return s;
 }
 
-extern "C" int d3d_gemm_rows64_silu_mul(const void* x, const void* w_gate_up, void* y, int M, int H, int K,
-                                        void* stream) {
-    if (M < 1 || M > 64 || H < 32 || H % 32 || K < gemm::TK || K % gemm::TK) return D3D_E_SHAPE;
-    if (!x || !w_gate_up || !y) return D3D_E_NULL;
-    if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w_gate_up) % 16) return D3D_E_UNSUPPORTED;
-    const dim3 grid(H / 32), block(gemm::NT);
-    const size_t lds = gemm::ST * gemm::STAGEB;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint16_t* xp = static_cast<const uint16_t*>(x);
-    const uint16_t* wp = static_cast<const uint16_t*>(w_gate_up);
-    uint16_t* yp = static_cast<uint16_t*>(y);
-    switch (K / gemm::TK) {
-#define D3D_ROWS64_SILU(n)                                                                                      \
-    case n:                                                                                                    \
-        hipLaunchKernelGGL((gemm::gemm_rows64_kernel<n, true>), grid, block, lds, s, xp, wp, yp, nullptr, M, 2 * H, K, \
-                           K);                                                                                 \
-        break;
-        D3D_ROWS64_SILU(8) D3D_ROWS64_SILU(16) D3D_ROWS64_SILU(24) D3D_ROWS64_SILU(32) D3D_ROWS64_SILU(48)
-        D3D_ROWS64_SILU(64)
-#undef D3D_ROWS64_SILU
-        default:
-            return D3D_E_UNSUPPORTED;
+namespace {
+
+struct Call {
+    const uint16_t *x, *w;
+    uint16_t* y;
+    float* parts;
+    int M, N, K, splits;
+    hipStream_t s;
+};
+
+template <int MR, int TN, int NW, int WC, int TK, int P, int STEPS>
+void launch(const Call& c) {
+    hipLaunchKernelGGL((gemm::rows_kernel<MR, TN, NW, WC, TK, P, STEPS, false>), dim3(c.N / TN, c.splits),
+                       dim3(NW * kWave), 0, c.s, c.x, c.w, c.y, c.parts, c.M, c.N, c.K, c.K / c.splits);
+}
+
+// Launches the variant built for this step count (steps of 128); false if
+// there is none.
+template <int MR, int TN, int NW, int WC, int TK, int P>
+bool launch_steps(const Call& c) {
+    constexpr int F = gemm::TK / TK;
+    switch (c.K / c.splits / gemm::TK) {
+        case 2: launch<MR, TN, NW, WC, TK, P, 2 * F>(c); return true;
+        case 4: launch<MR, TN, NW, WC, TK, P, 4 * F>(c); return true;
+        case 6: launch<MR, TN, NW, WC, TK, P, 6 * F>(c); return true;
+        case 8: launch<MR, TN, NW, WC, TK, P, 8 * F>(c); return true;
+        case 12: launch<MR, TN, NW, WC, TK, P, 12 * F>(c); return true;
+        case 16: launch<MR, TN, NW, WC, TK, P, 16 * F>(c); return true;
+        case 24: launch<MR, TN, NW, WC, TK, P, 24 * F>(c); return true;
+        case 32: launch<MR, TN, NW, WC, TK, P, 32 * F>(c); return true;
     }
+    if constexpr (MR <= 64) {
+        switch (c.K / c.splits / gemm::TK) {
+            case 1: launch<MR, TN, NW, WC, TK, P, F>(c); return true;
+            case 3: launch<MR, TN, NW, WC, TK, P, 3 * F>(c); return true;
+        }
+    }
+    return false;
+}
+
+int check(const void* x, const void* w, const void* y, const float* parts, int M, int max_rows, int N, int K,
+          int splits) {
+    if (M < 1 || M > max_rows || N < gemm::TN || N % gemm::TN || K < gemm::TK) return D3D_E_SHAPE;
+    if (splits < 1 || splits > gemm::kMaxSplits || K % (gemm::TK * splits)) return D3D_E_SHAPE;
+    if (!x || !w || (splits == 1 ? !y : !parts)) return D3D_E_NULL;
+    if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return D3D_E_UNSUPPORTED;
+    return D3D_OK;
+}
+
+}  // namespace
+
+extern "C" int d3d_gemm_rows64(const void* x, const void* w, void* y, float* parts, int M, int N, int K,
+                               int splits, void* stream) {
+    const int st = check(x, w, y, parts, M, 64, N, K, splits);
+    if (st != D3D_OK) return st;
+    const Call c{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), static_cast<uint16_t*>(y), parts,
+                 M, N, K, splits, static_cast<hipStream_t>(stream)};
+    const bool done = M <= 16   ? launch_steps<16, 64, 4, 4, 128, 2>(c)
+                      : M <= 32 ? launch_steps<32, 64, 4, 4, 128, 2>(c)
+                                : launch_steps<64, 64, 4, 4, 64, 3>(c);
+    if (!done)
+        hipLaunchKernelGGL(gemm::gemm_rows64_dma_kernel, dim3(N / gemm::TN, splits), dim3(gemm::NT),
+                           gemm::ST * gemm::STAGEB, c.s, c.x, c.w, c.y, parts, M, N, K, K / splits);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? D3D_OK : (int)err;
 }
 
-extern "C" int d3d_gemm_rows64(const void* x, const void* w, void* y, float* parts, int M, int N, int K,
-                               int splits, void* stream) {
-    if (M < 1 || M > 64 || N < gemm::TN || N % gemm::TN || K < gemm::TK) return D3D_E_SHAPE;
-    if (splits < 1 || splits > gemm::kMaxSplits || K % (gemm::TK * splits)) return D3D_E_SHAPE;
-    if (!x || !w || (splits == 1 ? !y : !parts)) return D3D_E_NULL;
-    if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(w) % 16) return D3D_E_UNSUPPORTED;
-    const dim3 grid(N / gemm::TN, splits), block(gemm::NT);
-    const size_t lds = gemm::ST * gemm::STAGEB;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const uint16_t* xp = static_cast<const uint16_t*>(x);
-    const uint16_t* wp = static_cast<const uint16_t*>(w);
-    uint16_t* yp = static_cast<uint16_t*>(y);
-    const int KR = K / splits;
-    switch (KR / gemm::TK) {
-#define D3D_ROWS64_STEPS(n) \
-    case n: hipLaunchKernelGGL(gemm::gemm_rows64_kernel<n>, grid, block, lds, s, xp, wp, yp, parts, M, N, K, KR); break;
-        D3D_ROWS64_STEPS(1) D3D_ROWS64_STEPS(2) D3D_ROWS64_STEPS(3) D3D_ROWS64_STEPS(4) D3D_ROWS64_STEPS(6)
-        D3D_ROWS64_STEPS(8) D3D_ROWS64_STEPS(12) D3D_ROWS64_STEPS(16) D3D_ROWS64_STEPS(24) D3D_ROWS64_STEPS(32)
-#undef D3D_ROWS64_STEPS
-        default:
-            hipLaunchKernelGGL(gemm::gemm_rows64_dma_kernel, grid, block, lds, s, xp, wp, yp, parts, M, N, K, KR);
-    }
+extern "C" int d3d_gemm_rows192(const void* x, const void* w, void* y, float* parts, int M, int N, int K, int splits,
+                                void* stream) {
+    if (M <= 64) return d3d_gemm_rows64(x, w, y, parts, M, N, K, splits, stream);
+    const int st = check(x, w, y, parts, M, gemm::kMaxRows, N, K, splits);
+    if (st != D3D_OK) return st;
+    const Call c{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), static_cast<uint16_t*>(y), parts,
+                 M, N, K, splits, static_cast<hipStream_t>(stream)};
+    if (!(M <= 128 ? launch_steps<128, 64, 8, 2, 64, 2>(c) : launch_steps<192, 64, 8, 2, 64, 2>(c)))
+        return D3D_E_UNSUPPORTED;
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? D3D_OK : (int)err;
 }

@@ -9,7 +9,7 @@
                          serving/vendor/ssd/layers/attention.py:21-22, one launch
 * ``silu_mul``        -- SiluAndMul (serving/vendor/ssd/layers/activation.py:6-14)
 * ``project``         -- the decoder layer's F.linear for blocks of at most
-                         64 rows (the qkv, o and down projections of a verify
+                         192 rows (the qkv, o and down projections of a verify
                          or draft block), by a weight-streaming HIP GEMM whose
                          K-split partials ``add_rmsnorm`` and
                          ``qk_rope_append`` sum on the way in
@@ -26,7 +26,12 @@ import torch.nn.functional as F
 
 from . import _lib
 
-ROWS64 = 64  # largest block project() runs on the HIP GEMM
+ROWS64 = 64  # largest block of d3d_gemm_rows64
+ROWS192 = 192  # largest block of d3d_gemm_rows192
+
+
+# k steps (of 128) per split that d3d_gemm_rows192 is built for above 64 rows.
+_STEPS192 = (2, 4, 6, 8, 12, 16, 24, 32)
 
 
 @dataclass(frozen=True)
@@ -58,8 +63,8 @@ Product = Union[torch.Tensor, SplitProduct]
 
 
 def rows64_splits(N: int, K: int) -> int:
-    """The split count project() runs d3d_gemm_rows64 with for a 64-row
-    block times weight [N, K], or 0 where it uses hipBLASLt instead.
+    """The split count project() runs d3d_gemm_rows192 with for a block
+    times weight [N, K], or 0 where it uses hipBLASLt instead.
 
     The kernel holds two workgroups per CU (256 CUs); its grid is N / 64
     column tiles times the splits.  Grids of 128 to 256 workgroups and of
@@ -69,7 +74,10 @@ def rows64_splits(N: int, K: int) -> int:
     draft gate-up at 192 14.8-16.2 against 15.7 us on its tuned library
     solution and 17.2-18.2 on the default one.  A round and a half (the
     24576 x 4096 target gate-up at 384: 48.0 against 46.9 us) and smaller
-    grids stay with hipBLASLt.
+    grids stay with hipBLASLt.  At 128 and 192 rows the same grids are ahead
+    by more (target qkv 19.7 against 25.7 us and 24.3 against 34.4, target
+    down 29.8 against 67.4 and 37.0 against 90.8); the one split of the
+    12288 x 2048 gate-up is even there (19.2 against 19.1, 23.7 against 25.9).
     """
     if N % 64 or K % 128:
         return 0
@@ -78,64 +86,76 @@ def rows64_splits(N: int, K: int) -> int:
     return splits if 128 <= grid <= 256 or grid == 512 else 0
 
 
-def project(x: torch.Tensor, weight: torch.Tensor) -> Product:
+def project(x: torch.Tensor, weight: torch.Tensor, max_rows: int = ROWS64) -> Product:
     """F.linear(x, weight) for bf16 x [M, K] and weight [N, K].
 
-    Contiguous, 16-byte aligned blocks of at most 64 rows with N % 64 == 0
-    and K % 128 == 0 run d3d_gemm_rows64 where rows64_splits says so; when
-    it splits K the result is a SplitProduct for add_rmsnorm or
-    qk_rope_append to consume.  Other shapes use F.linear (hipBLASLt).
+    Contiguous, 16-byte aligned blocks of at most ``max_rows`` (64 by default,
+    ROWS192 in the model's forwards) rows with N % 64 == 0
+    and K % 128 == 0 run d3d_gemm_rows192 where rows64_splits says so (above
+    64 rows only for the k-step counts it is built for); when it splits K the
+    result is a SplitProduct for add_rmsnorm or qk_rope_append to consume.
+    Other shapes use F.linear (hipBLASLt).
     """
     M, K = x.shape
     N = weight.shape[0]
-    if (M > ROWS64 or N % 64 or K % 128 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16
+    if (M > min(max_rows, ROWS192) or N % 64 or K % 128 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16
             or not x.is_contiguous() or not weight.is_contiguous()
             or x.data_ptr() % 16 or weight.data_ptr() % 16):  # the kernel's 16-byte row loads
         return F.linear(x, weight)
     dev = _lib.require_device(x, weight)
     lib = _lib.load()
     splits = rows64_splits(N, K)
-    if not splits:
+    if not splits or (M > ROWS64 and K // splits // 128 not in _STEPS192):
         return F.linear(x, weight)
     if splits == 1:
         y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
-        st = lib.d3d_gemm_rows64(x.data_ptr(), weight.data_ptr(), y.data_ptr(), None, M, N, K, 1, _lib.stream_ptr(dev))
-        _lib.check(st, "d3d_gemm_rows64")
+        st = lib.d3d_gemm_rows192(x.data_ptr(), weight.data_ptr(), y.data_ptr(), None, M, N, K, 1, _lib.stream_ptr(dev))
+        _lib.check(st, "d3d_gemm_rows192")
         return y
     parts = torch.empty(splits, M, N, dtype=torch.float32, device=dev)
-    st = lib.d3d_gemm_rows64(x.data_ptr(), weight.data_ptr(), None, parts.data_ptr(), M, N, K, splits,
-                             _lib.stream_ptr(dev))
-    _lib.check(st, "d3d_gemm_rows64")
+    st = lib.d3d_gemm_rows192(x.data_ptr(), weight.data_ptr(), None, parts.data_ptr(), M, N, K, splits,
+                              _lib.stream_ptr(dev))
+    _lib.check(st, "d3d_gemm_rows192")
     return SplitProduct(parts, splits)
 
 
 def rows64_silu_ok(H: int, K: int) -> bool:
     """Whether gate_up_silu runs the fused d3d_gemm_rows64_silu_mul for a
-    gate-up weight [2H, K] (its grid is 2H / 64 workgroups; the same grids
-    as rows64_splits, and the step counts the kernel is built for)."""
+    gate-up weight [2H, K] and at most 64 rows: grids of 128 to 512 workgroups
+    of 64 columns (above 256 in column tiles of 128 from 33 rows) and the step
+    counts the kernel is built for.  24576 x 4096, 16 rows: 43.1 us against
+    46.9 and a SiLU-mul of 3-5; 64 rows 46.5 against 50.3 and a SiLU-mul."""
     grid = 2 * H // 64
-    return H % 32 == 0 and K % 128 == 0 and K // 128 in (8, 16, 24, 32, 48, 64) and (128 <= grid <= 256 or grid == 512)
+    return (H % 32 == 0 and K % 128 == 0 and K // 128 in (8, 16, 24, 32, 48, 64) and 128 <= grid <= 512
+            and (grid <= 256 or H % 64 == 0))
+
+
+def rows_silu_ok(M: int, H: int, K: int) -> bool:
+    """rows64_silu_ok for M rows.  65-128 rows: grids of one round (12288 x
+    2048: 19.2 us against 19.1 and a SiLU-mul); 24576 x 4096 is behind there
+    (57-59 against 53.4 and 5).  129-192 rows: all (23.7 against 25.9, 60.9
+    against 64.9, before the SiLU-mul)."""
+    return M <= ROWS192 and rows64_silu_ok(H, K) and (not ROWS64 < M <= 128 or 2 * H // 64 <= 256)
 
 
 def gate_up_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """silu_mul(F.linear(x, weight)) for bf16 x [M, K] and a gate-up weight
     [2H, K] (gate rows, then up rows), the MLP's gate_up_proj + SiluAndMul.
 
-    Blocks of at most 64 rows whose shape rows64_silu_ok accepts run one
-    fused launch (d3d_gemm_rows64_silu_mul), equal bit for bit to
-    d3d_gemm_rows64 followed by silu_mul; others run F.linear (hipBLASLt)
-    and silu_mul."""
+    Blocks whose shape rows_silu_ok accepts run one fused launch
+    (d3d_gemm_rows192_silu_mul), equal bit for bit to d3d_gemm_rows192
+    followed by silu_mul; others run F.linear (hipBLASLt) and silu_mul."""
     M, K = x.shape
     H = weight.shape[0] // 2
-    if (M > ROWS64 or weight.shape[0] % 2 or not rows64_silu_ok(H, K) or x.dtype != torch.bfloat16
+    if (weight.shape[0] % 2 or not rows_silu_ok(M, H, K) or x.dtype != torch.bfloat16
             or weight.dtype != torch.bfloat16 or not x.is_contiguous() or not weight.is_contiguous()
             or x.data_ptr() % 16 or weight.data_ptr() % 16 or weight.shape[1] != K):
         return silu_mul(F.linear(x, weight))
     dev = _lib.require_device(x, weight)
     y = torch.empty(M, H, dtype=torch.bfloat16, device=dev)
-    st = _lib.load().d3d_gemm_rows64_silu_mul(x.data_ptr(), weight.data_ptr(), y.data_ptr(), M, H, K,
-                                              _lib.stream_ptr(dev))
-    _lib.check(st, "d3d_gemm_rows64_silu_mul")
+    st = _lib.load().d3d_gemm_rows192_silu_mul(x.data_ptr(), weight.data_ptr(), y.data_ptr(), M, H, K,
+                                               _lib.stream_ptr(dev))
+    _lib.check(st, "d3d_gemm_rows192_silu_mul")
     return y
 
 

@@ -217,11 +217,11 @@ class Qwen3PagedModel(torch.nn.Module):
         add + RMSNorm, QKV GEMM, fused q/k norm + RoPE + KV append, paged
         attention, O GEMM, fused add + RMSNorm, gate-up GEMM, fused SiLU-mul,
         down GEMM (the decoder layer of serving/vendor/ssd/models/qwen3.py).
-        Blocks of at most 64 tokens run the projections on the
+        Blocks of at most 192 tokens run the projections on the
         weight-streaming HIP GEMM where layers.project / gate_up_silu pick it
         (when ``rows64_gemm``: the QKV, O and down GEMMs, whose K-split
-        partials the next fused kernel sums, and the draft's gate-up with the
-        SiLU-mul fused in); the target's gate-up and larger blocks use
+        partials the next fused kernel sums, and the gate-up with the SiLU-mul
+        fused in, but for the target's at 65-128 rows); larger blocks use
         F.linear.
         """
         B, Q = ids.shape
@@ -231,7 +231,9 @@ class Qwen3PagedModel(torch.nn.Module):
         residual = F.embedding(ids.reshape(-1), self.embed)  # updated in place below
         hs = torch.empty_like(residual)
         x = None
-        proj = ly.project if self.rows64_gemm else F.linear
+        def proj(a, w):
+            return ly.project(a, w, ly.ROWS192) if self.rows64_gemm else F.linear(a, w)
+
         for li, L in enumerate(self.layers):
             ly.add_rmsnorm(x, residual, L["ln1"], s.eps, out=hs)
             qkv = proj(hs, L["qkv"])

@@ -528,6 +528,13 @@ int d3d_gemm_rows64(const void* x, const void* w, void* y, float* parts, int M, 
  */
 int d3d_gemm_rows64_silu_mul(const void* x, const void* w_gate_up, void* y, int M, int H, int K, void* stream);
 
+/* d3d_gemm_rows64 and d3d_gemm_rows64_silu_mul for blocks of at most 192 rows
+ * (the same kernels up to 64).  Above 64 rows d3d_gemm_rows192 takes K /
+ * splits / 128 in {2, 4, 6, 8, 12, 16, 24, 32} (D3D_E_UNSUPPORTED otherwise). */
+int d3d_gemm_rows192(const void* x, const void* w, void* y, float* parts, int M, int N, int K, int splits,
+                     void* stream);
+int d3d_gemm_rows192_silu_mul(const void* x, const void* w_gate_up, void* y, int M, int H, int K, void* stream);
+
 /* The split count d3d_gemm_rows64 is fastest with for an [N, K] weight (1 when N or K
  * is not a multiple of 64 or 128). */
 int d3d_gemm_rows64_splits(int N, int K);
