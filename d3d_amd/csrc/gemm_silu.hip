@@ -36,19 +36,32 @@ bool launch_steps(const SiluCall& c) {
 }
 
 // Column tiles of 64 while they make at most one round of 256 workgroups, or
-// up to 32 rows, where a workgroup takes little of a CU; else of 128, which
-// halve the reads of X.  Target gate-up, 24576 x 4096 (41.0 us at the copy
-// rate), us: 16 rows 43.1; 64 rows 51.5 with tiles of 64, 46.5 with 128; 192
-// rows 80.3 with 64, 60.9 with 128.
-bool wide_tile(int M, int H) { return M > 32 && H / 32 > 256 && H % 64 == 0; }
+// up to 32 rows, where a workgroup takes little of a CU; else of 96 where
+// those make a round, or of 128: fewer workgroups read X.  Target gate-up,
+// 24576 x 4096 (41.0 us at the copy rate), tiles of 64 / 96 / 128, us: 64 rows
+// 51.5 / 43.7 / 46.5 (hipBLASLt 49.5 and a SiLU-mul of 5), 128 rows 67.2 /
+// 50.6 / 57.0 (52.9), 192 rows 80.3 / 63.6 / 60.9 (60.4); 16 rows 43.1 with 64.
+int column_tile(int M, int H) {
+    if (M <= 32 || H / 32 <= 256) return 64;
+    if (M <= 128 && H % 48 == 0 && H / 48 <= 256) return 96;
+    return H % 64 == 0 ? 128 : 64;
+}
 
 int run(const SiluCall& c) {
-    bool done;
+    bool done = false;
+    const int tn = column_tile(c.M, c.H);
     if (c.M <= 16) done = launch_steps<16, 64, 4, 4, 128>(c);
     else if (c.M <= 32) done = launch_steps<32, 64, 4, 4, 128>(c);
-    else if (c.M <= 64) done = wide_tile(c.M, c.H) ? launch_steps<64, 128, 8, 4, 128>(c) : launch_steps<64, 64, 4, 4, 128>(c);
-    else if (c.M <= 128) done = launch_steps<128, 64, 8, 2, 64>(c);
-    else done = wide_tile(c.M, c.H) ? launch_steps<192, 128, 8, 4, 64>(c) : launch_steps<192, 64, 8, 2, 64>(c);
+    else if (c.M <= 64)
+        done = tn == 96    ? launch_steps<64, 96, 8, 2, 128>(c)
+               : tn == 128 ? launch_steps<64, 128, 8, 4, 128>(c)
+                           : launch_steps<64, 64, 4, 4, 128>(c);
+    else if (c.M <= 128)
+        done = tn == 96    ? launch_steps<128, 96, 4, 2, 64>(c)
+               : tn == 128 ? launch_steps<128, 128, 8, 4, 64>(c)
+                           : launch_steps<128, 64, 8, 2, 64>(c);
+    else
+        done = tn == 128 ? launch_steps<192, 128, 8, 4, 64>(c) : launch_steps<192, 64, 8, 2, 64>(c);
     if (!done) return D3D_E_UNSUPPORTED;
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? D3D_OK : (int)err;

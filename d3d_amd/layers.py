@@ -122,20 +122,22 @@ def project(x: torch.Tensor, weight: torch.Tensor, max_rows: int = ROWS64) -> Pr
 def rows64_silu_ok(H: int, K: int) -> bool:
     """Whether gate_up_silu runs the fused d3d_gemm_rows64_silu_mul for a
     gate-up weight [2H, K] and at most 64 rows: grids of 128 to 512 workgroups
-    of 64 columns (above 256 in column tiles of 128 from 33 rows) and the step
+    of 64 columns (above 256 in wider column tiles from 33 rows) and the step
     counts the kernel is built for.  24576 x 4096, 16 rows: 43.1 us against
-    46.9 and a SiLU-mul of 3-5; 64 rows 46.5 against 50.3 and a SiLU-mul."""
+    46.9 and a SiLU-mul of 3-5; 64 rows 43.7 against 49.5 and a SiLU-mul."""
     grid = 2 * H // 64
     return (H % 32 == 0 and K % 128 == 0 and K // 128 in (8, 16, 24, 32, 48, 64) and 128 <= grid <= 512
             and (grid <= 256 or H % 64 == 0))
 
 
 def rows_silu_ok(M: int, H: int, K: int) -> bool:
-    """rows64_silu_ok for M rows.  65-128 rows: grids of one round (12288 x
-    2048: 19.2 us against 19.1 and a SiLU-mul); 24576 x 4096 is behind there
-    (57-59 against 53.4 and 5).  129-192 rows: all (23.7 against 25.9, 60.9
-    against 64.9, before the SiLU-mul)."""
-    return M <= ROWS192 and rows64_silu_ok(H, K) and (not ROWS64 < M <= 128 or 2 * H // 64 <= 256)
+    """rows64_silu_ok for M rows.  65-128 rows: grids of one round of tiles of
+    64 or 96 columns (12288 x 2048: 19.2 us against 19.1 and a SiLU-mul; 24576
+    x 4096: 50.6 against 52.9 and 5; its tiles of 128 are behind, 57).  129-192
+    rows: all (23.7 against 25.9, 60.9 against 60.4-64.9, before the SiLU-mul)."""
+    if M > ROWS192 or not rows64_silu_ok(H, K):
+        return False
+    return not ROWS64 < M <= 128 or H // 32 <= 256 or (H % 48 == 0 and H // 48 <= 256)
 
 
 def gate_up_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

@@ -58,7 +58,7 @@ def test_every_step_count(M, K, splits):
     _check(y if splits == 1 else ly.SplitProduct(parts, splits).value(), x, w)
 
 
-@pytest.mark.parametrize("H,K", [(6144, 2048), (12288, 4096), (256, 1024), (8224, 1024)])
+@pytest.mark.parametrize("H,K", [(6144, 2048), (12288, 4096), (256, 1024), (8224, 1024), (12000, 1024)])
 @pytest.mark.parametrize("M", [16, 20, 64, 65, 128, 129, 192])
 def test_fused_gate_up_equals_the_two_kernels(H, K, M):
     lib = _lib.load()
