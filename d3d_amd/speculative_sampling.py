@@ -93,8 +93,10 @@ def _prep(t: torch.Tensor) -> torch.Tensor:
 
 
 def _outputs(B: int, K: int, dev: torch.device, posterior: bool = True):
-    return (torch.empty(B, dtype=torch.int32, device=dev), torch.empty(B, K, dtype=torch.uint8, device=dev),
-            torch.empty(B, dtype=torch.int64, device=dev), torch.empty(B, dtype=torch.uint8, device=dev),
+    # The kernels write 0 / 1 bytes: bool tensors as they are (converting them
+    # took two more launches of 2 us).
+    return (torch.empty(B, dtype=torch.int32, device=dev), torch.empty(B, K, dtype=torch.bool, device=dev),
+            torch.empty(B, dtype=torch.int64, device=dev), torch.empty(B, dtype=torch.bool, device=dev),
             torch.empty(B, K + 1, dtype=torch.int64, device=dev) if posterior else None)
 
 
@@ -162,7 +164,7 @@ def accept_fused(
         _lib.ptr(post), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev),
     )
     _lib.check(status, "d3d_accept_fused")
-    return AcceptOutput(accepted, mask.bool(), out_token, all_acc.bool(), post)
+    return AcceptOutput(accepted, mask, out_token, all_acc, post)
 
 
 def accept_fused_sparse(
@@ -223,7 +225,7 @@ def accept_fused_sparse(
         _lib.ptr(post), _lib.ptr(ws), ws.numel(), _lib.stream_ptr(dev),
     )
     _lib.check(status, "d3d_accept_fused_sparse")
-    return AcceptOutput(accepted, mask.bool(), out_token, all_acc.bool(), post)
+    return AcceptOutput(accepted, mask, out_token, all_acc, post)
 
 
 def _to_result(out: AcceptOutput) -> SpeculativeSampleResult:
