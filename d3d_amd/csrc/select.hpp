@@ -13,6 +13,8 @@
 namespace d3d {
 namespace filt {
 
+using rows::Scale;
+
 constexpr int NTF = 1024;              // threads per row workgroup
 constexpr int kWaves = NTF / kWave;    // 16
 constexpr int kIdBits = 18;            // ids < 2^18 in a support key
@@ -40,44 +42,6 @@ __device__ __forceinline__ float float_of(uint32_t k) {
     const uint32_t u = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
     return __uint_as_float(u);
 }
-
-// x / T, correctly rounded as the division is, in three multiply-adds: with
-// inv = 1 / T correctly rounded, q = x * inv is within one unit of the
-// quotient, r = x - q * T is exact, and q + r * inv rounds to x / T
-// (Markstein's theorem; it excludes a T whose mantissa is all ones).  Entries
-// whose intermediate values could leave the normal range, zeros, infinities
-// and NaN take the division.
-struct Scale {
-    float T, inv;
-    bool unit, fast;
-    __device__ __forceinline__ explicit Scale(float t)
-        : T(t), inv(1.0f / t), unit(t == 1.0f),
-          fast(t > 0x1p-20f && t < 0x1p40f && (__float_as_uint(t) & 0x7fffffu) != 0x7fffffu) {}
-    // x[] <- x[] / T.  The wave takes the division if any entry needs it: a
-    // branch per entry would leave no two entries' chains overlapping.
-    template <int LT>
-    __device__ __forceinline__ void tile(float (&x)[LT]) const {
-        if (unit) return;
-        if (fast) {
-            float z[LT];
-            bool odd = false;
-#pragma unroll
-            for (int l = 0; l < LT; ++l) {
-                const float q = x[l] * inv;
-                z[l] = __builtin_fmaf(__builtin_fmaf(-q, T, x[l]), inv, q);
-                // |x| outside [2^-60, 2^60)
-                odd |= (__float_as_uint(x[l]) & 0x7fffffffu) - 0x21800000u >= 0x3c000000u;
-            }
-            if (!__ballot(odd)) {
-#pragma unroll
-                for (int l = 0; l < LT; ++l) x[l] = z[l];
-                return;
-            }
-        }
-#pragma unroll
-        for (int l = 0; l < LT; ++l) x[l] = x[l] / T;
-    }
-};
 
 template <int DT>
 __device__ __forceinline__ float scaled(const void* row, int e, float T, bool unit) {
