@@ -18,6 +18,8 @@
 #include "d3d_common.hpp"
 #include "../../include/d3d_hip.h"
 
+#include <algorithm>
+
 namespace d3d {
 namespace paged {
 
@@ -48,6 +50,25 @@ __global__ __launch_bounds__(NT) void block_inputs_kernel(const int32_t* pool, i
     if (threadIdx.x == 0 && lens) lens[b] = start + Q;
 }
 
+// Up to kMaxCopies small buffers in one launch (a block step's static inputs:
+// token ids, positions, page tables, slots, lengths), 4 bytes per thread.
+// Each copy is a launch of its own that moves a few KB: a 4-layer verify step
+// went 691.9 -> 684.1 us (one request), 961.3 -> 952.6 (eight).
+constexpr int kMaxCopies = 8;
+
+struct Copies {
+    const uint32_t* src[kMaxCopies];
+    uint32_t* dst[kMaxCopies];
+    uint32_t words[kMaxCopies];
+};
+
+__global__ void copy_buffers_kernel(Copies c) {
+    const uint32_t* src = c.src[blockIdx.y];
+    uint32_t* dst = c.dst[blockIdx.y];
+    const uint32_t n = c.words[blockIdx.y];
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[i] = src[i];
+}
+
 }  // namespace paged
 }  // namespace d3d
 
@@ -64,6 +85,29 @@ extern "C" int d3d_block_inputs(const int32_t* page_pool, int pool_rows, int poo
     hipLaunchKernelGGL(paged::block_inputs_kernel, dim3(B), dim3(paged::NT), 0, static_cast<hipStream_t>(stream),
                        page_pool, pool_width, pool_rows, rows, starts, Q, width, page_size, tables_out, slots_out,
                        positions_out, context_lens_out);
+    const hipError_t err = hipGetLastError();
+    return err == hipSuccess ? D3D_OK : (int)err;
+}
+
+extern "C" int d3d_copy_buffers(int n, const void* const* src, void* const* dst, const size_t* bytes, void* stream) {
+    using namespace paged;
+    if (n < 0 || n > kMaxCopies) return D3D_E_SHAPE;
+    if (n == 0) return D3D_OK;
+    if (!src || !dst || !bytes) return D3D_E_NULL;
+    Copies c{};
+    size_t most = 0;
+    for (int i = 0; i < n; ++i) {
+        if (bytes[i] % 4 || bytes[i] / 4 > UINT32_MAX) return D3D_E_SHAPE;
+        if (bytes[i] && (!src[i] || !dst[i])) return D3D_E_NULL;
+        if ((uintptr_t)src[i] % 4 || (uintptr_t)dst[i] % 4) return D3D_E_UNSUPPORTED;
+        c.src[i] = static_cast<const uint32_t*>(src[i]);
+        c.dst[i] = static_cast<uint32_t*>(dst[i]);
+        c.words[i] = (uint32_t)(bytes[i] / 4);
+        most = std::max(most, bytes[i] / 4);
+    }
+    if (most == 0) return D3D_OK;
+    const int blocks = (int)std::min<size_t>((most + 255) / 256, 256);
+    hipLaunchKernelGGL(copy_buffers_kernel, dim3(blocks, n), dim3(256), 0, static_cast<hipStream_t>(stream), c);
     const hipError_t err = hipGetLastError();
     return err == hipSuccess ? D3D_OK : (int)err;
 }

@@ -28,6 +28,7 @@ attention over the prompt (any prompt length).
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
@@ -381,6 +382,9 @@ class BlockStep:
         self.tables = torch.zeros(B, width, dtype=torch.int32, device=dev)
         self.slots = torch.zeros(B * Q, dtype=torch.int64, device=dev)
         self.lens = torch.ones(B, dtype=torch.int32, device=dev)
+        self._static = (self.ids, self.pos, self.tables, self.slots, self.lens)
+        self._copies = (5, (ctypes.c_void_p * 5)(*(t.data_ptr() for t in self._static)),
+                        (ctypes.c_size_t * 5)(*(t.numel() * t.element_size() for t in self._static)))
         self.max_ctx = width * kv.page_size
         self.graph = None
         self.out = None
@@ -402,11 +406,18 @@ class BlockStep:
         return self.post(hidden, self.ids) if self.post is not None else None
 
     def _load(self, ids, pos, tables, slots, lens):
-        self.ids.copy_(ids, non_blocking=True)
-        self.pos.copy_(pos, non_blocking=True)
-        self.tables.copy_(tables, non_blocking=True)
-        self.slots.copy_(slots, non_blocking=True)
-        self.lens.copy_(lens, non_blocking=True)
+        src = (ids, pos, tables, slots, lens)
+        dst = self._static
+        if all(isinstance(s, torch.Tensor) and s.is_cuda and s.dtype == d.dtype and s.shape == d.shape
+               and s.device == d.device and s.is_contiguous() for s, d in zip(src, dst)):
+            # One launch for all five.
+            n, to, nbytes = self._copies
+            frm = (ctypes.c_void_p * n)(*(s.data_ptr() for s in src))
+            st = _lib.load().d3d_copy_buffers(n, frm, to, nbytes, _lib.stream_ptr(self.device))
+            _lib.check(st, "d3d_copy_buffers")
+            return
+        for d, s in zip(dst, src):
+            d.copy_(s, non_blocking=True)
 
     def __call__(self, ids, pos, tables, slots, lens):
         # Always under inference mode: torch keeps per-generator graph state

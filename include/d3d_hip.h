@@ -535,6 +535,13 @@ int d3d_gemm_rows192(const void* x, const void* w, void* y, float* parts, int M,
                      void* stream);
 int d3d_gemm_rows192_silu_mul(const void* x, const void* w_gate_up, void* y, int M, int H, int K, void* stream);
 
+/*
+ * Copies n <= 8 device buffers (bytes[i] from src[i] to dst[i], multiples of 4,
+ * 4-byte aligned, no destination overlapping another buffer) in one launch.
+ * The three arrays are host memory, read before the call returns.
+ */
+int d3d_copy_buffers(int n, const void* const* src, void* const* dst, const size_t* bytes, void* stream);
+
 /* The split count d3d_gemm_rows64 is fastest with for an [N, K] weight (1 when N or K
  * is not a multiple of 64 or 128). */
 int d3d_gemm_rows64_splits(int N, int K);
