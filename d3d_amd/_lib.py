@@ -87,6 +87,7 @@ SIGNATURES = {
     "d3d_sample_support_wide": (_I, [_P, _I, _I, _I64, _F, _I, _F, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "d3d_sample_support": (_I, [_P, _P, _I, _I, _F, _F, _P, _P, _P, _P, _P]),
     "d3d_add_rmsnorm": (_I, [_P, _P, _P, _P, _I, _I, _F, _P]),
+    "d3d_embed_rmsnorm": (_I, [_P, _P, _I64, _P, _P, _P, _I, _I, _F, _P]),
     "d3d_qk_rope_append": (
         _I,
         [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _I, _I64, _P],

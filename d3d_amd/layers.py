@@ -199,6 +199,25 @@ def add_rmsnorm(x: Optional[Product], residual: torch.Tensor, weight: torch.Tens
     return out
 
 
+def embed_rmsnorm(ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, eps: float):
+    """(residual, out) = (F.embedding(ids, table), RMSNorm(residual) * weight)
+    for ids [T] int64 and a contiguous bf16 table [V, H], in one launch."""
+    dev = _lib.require_device(ids, table, weight)
+    _bf16_rows(table, "table")
+    _bf16_rows(weight, "weight")
+    T, H = ids.numel(), table.shape[1]
+    if ids.dtype != torch.int64 or not ids.is_contiguous():
+        raise ValueError("ids must be contiguous int64")
+    if weight.numel() != H:
+        raise ValueError("weight must have one entry per hidden unit")
+    residual = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
+    out = torch.empty_like(residual)
+    st = _lib.load().d3d_embed_rmsnorm(ids.data_ptr(), table.data_ptr(), table.shape[0], residual.data_ptr(),
+                                       weight.data_ptr(), out.data_ptr(), T, H, float(eps), _lib.stream_ptr(dev))
+    _lib.check(st, "d3d_embed_rmsnorm")
+    return residual, out
+
+
 def qk_rope_append(qkv: Product, positions: torch.Tensor, q_norm: torch.Tensor, k_norm: torch.Tensor,
                    inv_freq: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                    slot_mapping: torch.Tensor, heads: int, kv_heads: int, eps: float, *, draft_rope: bool,

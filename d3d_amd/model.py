@@ -229,14 +229,16 @@ class Qwen3PagedModel(torch.nn.Module):
         s = self.shape
         Hq, Hkv, d = s.heads, s.kv_heads, s.head_dim
         pos = positions.reshape(-1)
-        residual = F.embedding(ids.reshape(-1), self.embed)  # updated in place below
-        hs = torch.empty_like(residual)
+        # The lookup with the first norm; residual and hs are updated in place below.
+        first = self.layers[0]["ln1"] if self.layers else self.norm
+        residual, hs = ly.embed_rmsnorm(ids.reshape(-1).to(torch.int64).contiguous(), self.embed, first, s.eps)
         x = None
         def proj(a, w):
             return ly.project(a, w, ly.ROWS192) if self.rows64_gemm else F.linear(a, w)
 
         for li, L in enumerate(self.layers):
-            ly.add_rmsnorm(x, residual, L["ln1"], s.eps, out=hs)
+            if li:
+                ly.add_rmsnorm(x, residual, L["ln1"], s.eps, out=hs)
             qkv = proj(hs, L["qkv"])
             q = ly.qk_rope_append(qkv, pos, L["qn"], L["kn"], self.inv_freq, kv.k[li], kv.v[li], slot_mapping,
                                   Hq, Hkv, s.eps, draft_rope=self.draft)

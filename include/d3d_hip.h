@@ -547,6 +547,16 @@ int d3d_copy_buffers(int n, const void* const* src, void* const* dst, const size
 int d3d_gemm_rows64_splits(int N, int K);
 
 /*
+ * The embedding lookup and the first layer's RMSNorm in one launch: residual
+ * [T, H] = table[ids] (ids [T] int64 in [0, vocab), table [vocab, H] bf16),
+ * out = RMSNorm(residual) * weight as d3d_add_rmsnorm with x NULL.  An id
+ * outside the table traps, as torch's lookup does.  H % 8 == 0, H <= 8192;
+ * table, residual, weight and out 16-byte aligned.
+ */
+int d3d_embed_rmsnorm(const int64_t* ids, const void* table, int64_t vocab, void* residual, const void* weight,
+                      void* out, int T, int H, float eps, void* stream);
+
+/*
  * d3d_add_rmsnorm with x given as the partials of d3d_gemm_rows64:
  * x[t, i] = bf16(sum over s in order of parts[s, t, i]), parts
  * [splits, T, H] fp32, 16-byte aligned.
