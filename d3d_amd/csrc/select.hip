@@ -804,8 +804,17 @@ __global__ __launch_bounds__(NT) void nucleus_gather_kernel(SelParams P) {
     const NucRec rec = find_bin(P, n, M, s_part, &s_rec, s_fine);
     if (p == 0 && threadIdx.x == 0) P.rec[n] = rec;
     const void* row = rows::row_ptr<DT>(P.logits, n, P.V);
-    const Scale scale(P.T);
     if (rec.bin < 0) return;
+    const Scale scale(P.T);
+    // The bin's entries lie in (M - (bin + 1) / 32, M - bin / 32] T; a range of
+    // x widened by more than the roundings of M - z, z = x / T and this
+    // product is tested first, and only a wave with an entry in it scales that
+    // entry (a few of 64 in a bin's worth of a row).
+    const float z_hi = M - (float)rec.bin / kBinScale, z_lo = z_hi - 1.f / kBinScale;
+    const float pad = (fabsf(M) + 32.f) * P.T * 0x1p-18f;
+    const float x_mid = (0.5f * z_hi + 0.5f * z_lo) * P.T;
+    // Out of range: every entry is taken for near.
+    const float x_half = fabsf(x_mid) < INFINITY ? (0.5f / kBinScale) * P.T + pad : INFINITY;
     uint64_t* list = P.list + (size_t)n * kMaxSel;
     const int c1 = min((p + 1) * P.span, P.C);
     for (int c = p * P.span; c < c1; ++c) {
@@ -813,9 +822,15 @@ __global__ __launch_bounds__(NT) void nucleus_gather_kernel(SelParams P) {
         float x[kGroup];
         rows::load_tile<DT, VEC, false, kGroup>(row, P.V, first, NT * E, -INFINITY, x);
         uint32_t hits = 0;  // bit l: entry l lies in the crossing bin
-        scale.tile(x);
 #pragma unroll
-        for (int l = 0; l < kGroup; ++l) hits |= (mass_bin(M - x[l]) == rec.bin ? 1u : 0u) << l;
+        for (int l = 0; l < kGroup; ++l) {
+            const bool near = !(fabsf(x[l] - x_mid) > x_half);
+            if (!__ballot(near)) continue;
+            float z[1] = {x[l]};
+            scale.tile(z);
+            x[l] = z[0];
+            hits |= (near && mass_bin(M - z[0]) == rec.bin ? 1u : 0u) << l;
+        }
         // One slot reservation per wave that holds such entries.
         const uint32_t cnt = __popc(hits);
         if (__ballot(cnt != 0)) {
@@ -847,8 +862,12 @@ __global__ __launch_bounds__(NTF) void nucleus_finish_kernel(SelParams P) {
     const int n = blockIdx.x;
     const bool unit = P.T == 1.0f;
     const void* row = rows::row_ptr<DT>(P.logits, n, P.V);
+    // The record, the count and this thread's first gathered entry load
+    // together (the list has kMaxSel slots, whatever they hold).
     const NucRec rec = P.rec[n];
-    const uint32_t m = rec.bin < 0 ? 0u : P.counter[n];
+    const uint32_t counted = P.counter[n];
+    const uint64_t key0 = P.list[(size_t)n * kMaxSel + threadIdx.x];
+    const uint32_t m = rec.bin < 0 ? 0u : counted;
     if (m > (uint32_t)kMaxSel) {
         filter_row_general<DT>(P, row, n, rec.M, unit, sc);
         return;
@@ -883,8 +902,8 @@ __global__ __launch_bounds__(NTF) void nucleus_finish_kernel(SelParams P) {
         }
         __syncthreads();
         for (int i = threadIdx.x; i < (int)m; i += NTF) {
-            const uint64_t w = weight_fx(key_value(src[i]), rec.M);
-            if (w) atomicAdd(&s_sub[sub_of(src[i])], (unsigned long long)w);
+            const uint64_t key = i < NTF ? key0 : src[i], w = weight_fx(key_value(key), rec.M);
+            if (w) atomicAdd(&s_sub[sub_of(key)], (unsigned long long)w);
         }
         __syncthreads();
         uint64_t tot;
@@ -894,14 +913,16 @@ __global__ __launch_bounds__(NTF) void nucleus_finish_kernel(SelParams P) {
         __syncthreads();
         const int b = sc.s.i[0];
         if ((int)threadIdx.x == b) sc.s.base = incl - mine;
-        for (int i = threadIdx.x; i < (int)m; i += NTF)
-            if (sub_of(src[i]) == b) list[atomicAdd(&sc.s.n_cand, 1u)] = src[i];
+        for (int i = threadIdx.x; i < (int)m; i += NTF) {
+            const uint64_t key = i < NTF ? key0 : src[i];
+            if (sub_of(key) == b) list[atomicAdd(&sc.s.n_cand, 1u)] = key;
+        }
         __syncthreads();
         const int m2 = (int)sc.s.n_cand;
         const uint64_t above = sc.s.base;
         pad_and_sort(list, m2, 0, sc.s.rank);
         // The part's mass crosses the target, so one of its entries does.
-        const int at = min(first_crossing(list, m2, rec.M, above, rec.target, sc), m2 - 1);
+        const int at = max(min(first_crossing(list, m2, rec.M, above, rec.target, sc), m2 - 1), 0);
         cut = list[at];
         zf = key_value(cut);
         lim = (int)(cut & ((1ull << kIdBits) - 1));
@@ -913,7 +934,7 @@ __global__ __launch_bounds__(NTF) void nucleus_finish_kernel(SelParams P) {
     if (!P.tok) return;
     __syncthreads();
     for (int i = threadIdx.x; i < (int)m; i += NTF) {
-        const uint64_t key = src[i], w = key <= cut ? weight_fx(key_value(key), rec.M) : 0;
+        const uint64_t key = i < NTF ? key0 : src[i], w = key <= cut ? weight_fx(key_value(key), rec.M) : 0;
         const int c = (int)(key & ((1ull << kIdBits) - 1)) / (kChunk * P.span);
         if (w) atomicAdd((unsigned long long*)&sc.s.mass[c], (unsigned long long)w);
     }

@@ -95,7 +95,7 @@ __device__ __forceinline__ uint64_t weight_fx(float z, float M) {
     // NaN (and +inf against itself) carries no mass; -inf gives exp = 0.  No
     // branch, so that the chains of a thread's entries overlap.
     const float d = z - M;
-    const float e = expf(fminf(d, 0.f));
+    const float e = rows::exp_nonpos(fminf(d, 0.f));
     // floor(e * 2^40): both halves of the 24-bit product are exact.
     const float f = d <= 0.f ? e * (float)kFix : 0.f;
     const uint32_t hi = (uint32_t)(f * 0x1p-32f);
