@@ -39,9 +39,12 @@
 // sub-tiles at a time, the operand layout of P^T in O^T = V^T P^T, so
 // probabilities never leave registers, and the O^T accumulators keep each
 // lane on the query row whose softmax statistics it holds (rescaling and
-// normalising need no cross-lane moves).  V is read 4 columns at a time (one
-// 8-byte LDS read serves four 16-dim output tiles): tile (h, q) holds dim
-// 64h + 4j + q in accumulator row j.  Online softmax runs in the log2
+// normalising need no cross-lane moves).  V is read from LDS with the
+// transposing 16-bit read, which hands each lane its four tokens of one dim:
+// two reads and no other instruction per operand (reading rows and permuting
+// halves took 64 v_perm_b32 per tile and wave: batch-8 verify call 26.6 -> 25.5
+// us, a prefill's attention over 7,800 tokens 372 -> 326 us a layer, the same
+// bits).  Online softmax runs in the log2
 // domain.  With more than one split, (m, l, O) partials go to the workspace
 // and a combine kernel merges them.
 #include "d3d_common.hpp"
@@ -74,6 +77,16 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// Transposing LDS read (ds_read_b64_tr_b16): each group of 16 lanes reads a 4 x
+// 16 block of 16-bit entries, lane i giving the address of row i / 4, columns
+// 4 (i % 4) .. + 3, and receives column i of the four rows.
+__device__ __forceinline__ u32x2 lds_read_tr(const char* p) {
+    return __builtin_bit_cast(
+        u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(const __attribute__((address_space(3))) char*)p));
+}
 
 struct Params {
     const uint16_t* q;
@@ -274,7 +287,7 @@ __device__ __forceinline__ void store_tile(char* lds, const u32x4 (&reg)[2 * TIL
 // counts the compiler reaches, four-wave workgroups run three per CU.
 // UPG: pages are a power of two of at least 4 tokens (wave-uniform page ids).
 // RT: row tiles of 16 per wave.  With RT = 2 each K fragment and each
-// permuted V operand read from LDS feeds two MFMAs (blocks of more than 64
+// transposed V operand read from LDS feeds two MFMAs (blocks of more than 64
 // rows per KV head: the packed draft block).
 template <int NW, int MODE, bool UPG, int RT>
 __global__ __launch_bounds__(NW * 64, 2) void attn_split_kernel(Params P) {
@@ -560,32 +573,18 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_split_kernel(Params P) {
                 pop[rt] = __builtin_bit_cast(bf16x8, pv);
             }
 #pragma unroll
-            for (int h = 0; h < D / 64; ++h) {
-                // V rows of the 8 token slots, 4 columns 64h + 4*c16 .. +3 each.
-                u32x2 vr[8];
+            for (int n = 0; n < D / 16; ++n) {
+                // A = V^T: lane l row dim 16n + l%16, its 8 token slots (32mp +
+                // 4*g4 + r, then 16 further) by two transposing reads.  B =
+                // P^T, lane l column = query row l%16, so the accumulator's
+                // rows are dims and its columns query rows.
+                const char* va16 = vl + (32 * mp + 4 * g4 + (c16 >> 2)) * ROWB_V + (16 * n + 4 * (c16 & 3)) * 2;
+                const u32x2 lo = lds_read_tr(va16), hi = lds_read_tr(va16 + 16 * ROWB_V);
+                const u32x4 vw = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
-                for (int kk = 0; kk < 8; ++kk) {
-                    const int t = 32 * mp + 16 * (kk >> 2) + 4 * g4 + (kk & 3);
-                    vr[kk] = *reinterpret_cast<const u32x2*>(vl + t * ROWB_V + (64 * h + 4 * c16) * 2);
-                }
-#pragma unroll
-                for (int qq = 0; qq < 4; ++qq) {
-                    // Column qq of each row: low or high half of word qq/2.
-                    const uint32_t sel = (qq & 1) ? 0x07060302u : 0x05040100u;
-                    const int word = qq >> 1;
-                    const u32x4 vw = {__builtin_amdgcn_perm(vr[1][word], vr[0][word], sel),
-                                      __builtin_amdgcn_perm(vr[3][word], vr[2][word], sel),
-                                      __builtin_amdgcn_perm(vr[5][word], vr[4][word], sel),
-                                      __builtin_amdgcn_perm(vr[7][word], vr[6][word], sel)};
-                    // O^T = V^T P^T: the same registers with the operands
-                    // swapped (A = V^T, lane l row dim 64h + 4(l%16) + qq;
-                    // B = P^T, lane l column = query row l%16), so the
-                    // accumulator rows are dims and its columns query rows.
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt)
-                        o[rt][4 * h + qq] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf16x8, vw), pop[rt], o[rt][4 * h + qq], 0, 0, 0);
-                }
+                for (int rt = 0; rt < RT; ++rt)
+                    o[rt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vw), pop[rt], o[rt][n],
+                                                                     0, 0, 0);
             }
         }
     };
@@ -643,22 +642,20 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_split_kernel(Params P) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) l_run[rt] = xor32_sum(xor16_sum(l_run[rt]));
 
-    // Lane (g4, c16) holds row c16 of row tile rt at dims 64h + 16 g4 + 4r +
-    // qq in o[rt][4h + qq][r]: four consecutive dims per (h, r).
+    // Lane (g4, c16) holds row c16 of row tile rt at dims 16n + 4 g4 + r in
+    // o[rt][n][r]: four consecutive dims per n.
     if (nsplit == 1) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const float inv = l_run[rt] > 0.f ? 1.f / l_run[rt] : 0.f;
             if (row_ok[rt]) {
-                uint16_t* dst = P.out + (((size_t)b * P.Q + qi[rt]) * P.Hq + head[rt]) * D + 16 * g4;
+                uint16_t* dst = P.out + (((size_t)b * P.Q + qi[rt]) * P.Hq + head[rt]) * D + 4 * g4;
 #pragma unroll
-                for (int h = 0; h < D / 64; ++h)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const u32x2 v = {pack_bf16x2(o[rt][4 * h + 0][r] * inv, o[rt][4 * h + 1][r] * inv),
-                                         pack_bf16x2(o[rt][4 * h + 2][r] * inv, o[rt][4 * h + 3][r] * inv)};
-                        *reinterpret_cast<u32x2*>(dst + 64 * h + 4 * r) = v;
-                    }
+                for (int n = 0; n < D / 16; ++n) {
+                    const u32x2 v = {pack_bf16x2(o[rt][n][0] * inv, o[rt][n][1] * inv),
+                                     pack_bf16x2(o[rt][n][2] * inv, o[rt][n][3] * inv)};
+                    *reinterpret_cast<u32x2*>(dst + 16 * n) = v;
+                }
             }
         }
     } else {
@@ -682,13 +679,11 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_split_kernel(Params P) {
             const float down = __uint_as_float((uint32_t)(127 - e) << 23) * inv;  // 2^-e / l
             if (row[rt] < P.M) {
 #pragma unroll
-                for (int h = 0; h < D / 64; ++h)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const h16x4 v = {(_Float16)(o[rt][4 * h + 0][r] * down), (_Float16)(o[rt][4 * h + 1][r] * down),
-                                         (_Float16)(o[rt][4 * h + 2][r] * down), (_Float16)(o[rt][4 * h + 3][r] * down)};
-                        *reinterpret_cast<h16x4*>(po + (size_t)row[rt] * D + 64 * h + 16 * g4 + 4 * r) = v;
-                    }
+                for (int n = 0; n < D / 16; ++n) {
+                    const h16x4 v = {(_Float16)(o[rt][n][0] * down), (_Float16)(o[rt][n][1] * down),
+                                     (_Float16)(o[rt][n][2] * down), (_Float16)(o[rt][n][3] * down)};
+                    *reinterpret_cast<h16x4*>(po + (size_t)row[rt] * D + 16 * n + 4 * g4) = v;
+                }
             }
             if (g4 == 0 && row_ok[rt])
                 pml[row[rt]] = make_float4(m_run[rt], l_run[rt], __uint_as_float((uint32_t)(127 + e) << 23), 0.f);
