@@ -160,7 +160,10 @@ def require_device(*tensors: Optional[torch.Tensor]) -> torch.device:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (0.1 us; a torch.cuda.Stream object for it
+    takes 1.5, twice in every call)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 _workspaces: dict = {}
