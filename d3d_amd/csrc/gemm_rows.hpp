@@ -14,31 +14,28 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // Rows the kernels take in all.
 constexpr int kMaxRows = 192;
 
-// One workgroup of NW waves (WC of them across the tile's columns), P k steps
-// of TK in flight in registers, STEPS steps in all; the lane's source rows and
-// LDS slots: global 16-byte chunk (lane % chunks) ^ (row & 7) of a tile row
-// goes to LDS chunk lane % chunks.
-//
-// SILU: W is a gate-up weight [2 H, K] (gate rows, then up rows) and Y
-// [M, H] = silu(bf16(X Wg^T)) * bf16(X Wu^T), each product rounded as the
-// bf16 GEMM output would be, then evaluated as d3d_silu_mul does.  Tile t
-// stands for output columns TN/2 t .. TN/2 t + TN/2 - 1: tile row 16 w + c is
-// the gate row of column TN/2 t + 8 w + c (c < 8) or the up row of column
-// TN/2 t + 8 w + c - 8, so a lane's gate and up products of one column sit in
-// lanes c and c + 8 of its 16-lane row.
-template <int MR, int TN, int NW, int WC, int TK, int P, int STEPS, bool SILU>
-__global__ __launch_bounds__(NW * kWave) void rows_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                          uint16_t* __restrict__ y, float* __restrict__ parts, int M,
-                                                          int N, int K, int KR) {
+// Bytes of LDS the main loop needs.
+template <int MR, int TN, int TK>
+constexpr int rows_lds() { return 2 * (TN + MR) * TK * 2; }
+
+// The main loop of a workgroup of NW waves (WC of them across the tile's TN
+// columns): acc[a][b] += X[rows, kb ..] W[wrow(0 .. TN - 1), kb ..]^T over STEPS
+// k steps of TK, P of them in flight in registers.  Wave wv holds rows ar0 +
+// 16a, columns bc0 + 16b, with ar0 = (wv / WC) (MR / WR), bc0 = (wv % WC) (TN / WC).
+// The lane's source rows and LDS slots: global 16-byte chunk (lane % chunks) ^
+// (row & 7) of a tile row goes to LDS chunk lane % chunks.  Rows of X past M
+// repeat the last one.
+template <int MR, int TN, int NW, int WC, int TK, int P, int STEPS, typename WRow>
+__device__ __forceinline__ void rows_main_loop(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M,
+                                               int K, int kb, char* smem, WRow&& wrow,
+                                               f32x4 (&acc)[MR * WC / NW / 16][TN / WC / 16]) {
     constexpr int RB = TK * 2, CPRW = RB / 16, RPIW = kWave / CPRW;  // bytes, 16-byte chunks of a tile row
     constexpr int WT = TN * RB, XT = MR * RB, STAGE = WT + XT;
     constexpr int NWL = WT / 1024 / NW, NXL = XT / 1024 / NW;  // load instructions per wave
     constexpr int WR = NW / WC, AR = MR / WR / 16, BC = TN / WC / 16;
     static_assert(AR * WR * 16 == MR && BC * WC * 16 == TN && NWL * NW * 1024 == WT && NXL * NW * 1024 == XT, "tile");
-    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int c16 = lane & 15, g4 = lane >> 4;
-    const int n0 = blockIdx.x * TN, kb = blockIdx.y * KR;
     const int lr = lane / CPRW, lc = lane % CPRW;
     const uint16_t* wsrc[NWL];
     const uint16_t* xsrc[NXL];
@@ -46,12 +43,7 @@ __global__ __launch_bounds__(NW * kWave) void rows_kernel(const uint16_t* __rest
 #pragma unroll
     for (int j = 0; j < NWL; ++j) {
         const int r = (wv * NWL + j) * RPIW + lr, q = lc ^ (r & 7);
-        int row = n0 + r;
-        if constexpr (SILU) {
-            const int col = TN / 2 * blockIdx.x + 8 * (r >> 4) + (r & 7);
-            row = (r & 8) ? N / 2 + col : col;
-        }
-        wsrc[j] = w + (size_t)row * K + kb + 8 * q;
+        wsrc[j] = w + (size_t)wrow(r) * K + kb + 8 * q;
         wofs[j] = r * RB + lc * 16;
     }
 #pragma unroll
@@ -68,7 +60,6 @@ __global__ __launch_bounds__(NW * kWave) void rows_kernel(const uint16_t* __rest
 #pragma unroll
         for (int j = 0; j < NXL; ++j) rx[sl][j] = *reinterpret_cast<const u32x4*>(xsrc[j] + st * TK);
     };
-    f32x4 acc[AR][BC];
 #pragma unroll
     for (int a = 0; a < AR; ++a)
 #pragma unroll
@@ -110,6 +101,33 @@ __global__ __launch_bounds__(NW * kWave) void rows_kernel(const uint16_t* __rest
                         __builtin_bit_cast(bf16x8, ax[a]), __builtin_bit_cast(bf16x8, bw[b]), acc[a][b], 0, 0, 0);
         }
     }
+}
+
+// SILU: W is a gate-up weight [2 H, K] (gate rows, then up rows) and Y
+// [M, H] = silu(bf16(X Wg^T)) * bf16(X Wu^T), each product rounded as the
+// bf16 GEMM output would be, then evaluated as d3d_silu_mul does.  Tile t
+// stands for output columns TN/2 t .. TN/2 t + TN/2 - 1: tile row 16 w + c is
+// the gate row of column TN/2 t + 8 w + c (c < 8) or the up row of column
+// TN/2 t + 8 w + c - 8, so a lane's gate and up products of one column sit in
+// lanes c and c + 8 of its 16-lane row.
+template <int MR, int TN, int NW, int WC, int TK, int P, int STEPS, bool SILU>
+__global__ __launch_bounds__(NW * kWave) void rows_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                          uint16_t* __restrict__ y, float* __restrict__ parts, int M,
+                                                          int N, int K, int KR) {
+    constexpr int WR = NW / WC, AR = MR / WR / 16, BC = TN / WC / 16;
+    __shared__ __attribute__((aligned(16))) char smem[rows_lds<MR, TN, TK>()];
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    const int c16 = lane & 15, g4 = lane >> 4;
+    const int n0 = blockIdx.x * TN, ar0 = (wv / WC) * (MR / WR), bc0 = (wv % WC) * (TN / WC);
+    f32x4 acc[AR][BC];
+    rows_main_loop<MR, TN, NW, WC, TK, P, STEPS>(
+        x, w, M, K, (int)blockIdx.y * KR, smem,
+        [&](int r) {
+            if constexpr (!SILU) return n0 + r;
+            const int col = TN / 2 * (int)blockIdx.x + 8 * (r >> 4) + (r & 7);
+            return (r & 8) ? N / 2 + col : col;
+        },
+        acc);
     // Lane (c16, g4) holds rows 16a + 4 g4 + r of column 16b + c16: bf16 into
     // Y (one split) or the fp32 partial of split blockIdx.y.
 #pragma unroll

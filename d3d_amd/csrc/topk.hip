@@ -30,6 +30,7 @@
 // 24.8, k = 4 30.7 / 27.1, k = 8 56.1 / 26.8; at 1,088 bf16 rows k = 4 161 /
 // 176, k = 8 235 / 176; one bf16 row k = 8 16.0 / 20.5.
 #include "d3d_common.hpp"
+#include "gemm_rows.hpp"
 #include "rowstats.hpp"
 #include "select.hpp"
 #include "../../include/d3d_hip.h"
@@ -550,6 +551,114 @@ __global__ __launch_bounds__(NT, 2) void lmhead_partial_xlds_kernel(LmParams P) 
     lmhead_epilogue<KK>(P, acc, slice, row0, reinterpret_cast<uint16_t*>(smem));
 }
 
+// The LM head on the weight-streaming main loop of gemm_rows.hpp, for H of
+// 2048 and 4096: the weight goes to LDS in whole 128- or 256-byte row segments
+// instead of to registers in 64-byte pieces of 16 rows, which stream at 4.1 of
+// 5.5 TB/s.  Slices of 128 weight rows, four waves, three workgroups per CU (a
+// slice's epilogue beside the others' streams).  The products and the bf16
+// logits are those of the kernels above; the records are merged the same way.
+// 64 rows, k = 2, 151,936 x 2048 (127 us at the copy rate): 171 -> 117 us, the
+// whole call 166 -> 131.
+constexpr int kRowCols = 128;  // weight rows per workgroup
+
+template <int KK, int MR, int TK, int STEPS>
+__global__ __launch_bounds__(NT) void lmhead_rows_kernel(LmParams P) {
+    constexpr int AR = MR / 16, BC = kRowCols / 4 / 16;  // four waves across the columns
+    constexpr int STRIDE = kRowCols + 8;                 // bf16 entries per LDS row (16-byte pad)
+    constexpr int TPR = NT / MR, PER = kRowCols / TPR;   // epilogue threads per row, columns each
+    constexpr int LDS = gemm::rows_lds<MR, kRowCols, TK>();
+    static_assert(MR * STRIDE * 2 <= LDS, "the logits reuse the tiles");
+    __shared__ __attribute__((aligned(16))) char smem[LDS];
+    const int slice = blockIdx.x, row0 = blockIdx.y * MR;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int c16 = lane & 15, g4 = lane >> 4;
+    gemm::f32x4 acc[AR][BC];
+    gemm::rows_main_loop<MR, kRowCols, 4, 4, TK, 2, STEPS>(
+        P.x + (size_t)row0 * P.H, P.w, P.T - row0, P.H, 0, smem,
+        [&](int r) { return min(slice * kRowCols + r, P.V - 1); }, acc);
+    uint16_t* s_log = reinterpret_cast<uint16_t*>(smem);
+    __syncthreads();  // every wave is done with the tiles
+#pragma unroll
+    for (int a = 0; a < AR; ++a)
+#pragma unroll
+        for (int b = 0; b < BC; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                s_log[(16 * a + 4 * g4 + r) * STRIDE + w * (kRowCols / 4) + 16 * b + c16] =
+                    f32_to_bf16_bits(acc[a][b][r]);
+    __syncthreads();
+    // TPR threads per hidden row, PER consecutive slice columns each.
+    const int row = threadIdx.x / TPR, q = threadIdx.x % TPR;
+    const int vbase = slice * kRowCols + PER * q;
+    const int nvalid = min(PER, P.V - vbase);  // may be <= 0 in the last slice
+    const uint16_t* src = &s_log[row * STRIDE + PER * q];
+    float tv[KK], xs[PER];
+    int ti[KK];
+#pragma unroll
+    for (int p = 0; p < KK; ++p) {
+        tv[p] = -INFINITY;
+        ti[p] = INT_MAX;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j8 = 0; j8 < PER; j8 += 8) {
+        float t[8];
+        unpack16<kBF16>(*reinterpret_cast<const u32x4*>(src + j8), t);
+#pragma unroll
+        for (int h = 0; h < 8; ++h) {
+            const int j = j8 + h;
+            xs[j] = j < nvalid ? t[h] : -INFINITY;
+            mx = fmaxf(mx, xs[j]);
+            // Ids rise with j, so an equal value never displaces an earlier one.
+            if (j < nvalid && xs[j] > tv[KK - 1]) list_insert<KK>(tv, ti, xs[j], vbase + j);
+        }
+    }
+    // Merge the row's threads (neighbouring lanes); partners end with the same list.
+#pragma unroll
+    for (int o = 1; o < TPR; o <<= 1) {
+        float ov[KK];
+        int oi[KK];
+#pragma unroll
+        for (int p = 0; p < KK; ++p) {
+            ov[p] = __shfl_xor(tv[p], o, kWave);
+            oi[p] = __shfl_xor(ti[p], o, kWave);
+        }
+#pragma unroll
+        for (int p = 0; p < KK; ++p) list_insert<KK>(tv, ti, ov[p], oi[p]);
+        mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
+    }
+    float se = 0.f;
+    if (mx != -INFINITY) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (j < nvalid) se += expf(xs[j] - mx);
+    }
+#pragma unroll
+    for (int o = 1; o < TPR; o <<= 1) se += __shfl_xor(se, o, kWave);
+    const int grow = row0 + row;
+    if (q == 0 && grow < P.T) {
+        Cand* dst = P.cand + ((size_t)grow * P.C + slice) * P.k;
+#pragma unroll
+        for (int p = 0; p < KK; ++p)
+            if (p < P.k) dst[p] = Cand{tv[p], ti[p]};
+        P.lse[(size_t)grow * P.C + slice] = make_float2(mx, se);
+    }
+}
+
+template <int KK>
+static void launch_lmhead_rows(const LmParams& L, hipStream_t s) {
+    // Up to 16 rows in a 16-row tile (most of the 64-row tile's X loads and
+    // MFMAs would be repeats).
+    if (L.T <= 16) {
+        if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 16, 128, 16>), dim3(L.C), dim3(NT), 0, s, L);
+        else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 16, 128, 32>), dim3(L.C), dim3(NT), 0, s, L);
+        return;
+    }
+    const dim3 grid(L.C, (L.T + 63) / 64);
+    if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 64, 64, 32>), grid, dim3(NT), 0, s, L);
+    else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 64, 64, 64>), grid, dim3(NT), 0, s, L);
+}
+
 }  // namespace topk
 }  // namespace d3d
 
@@ -620,13 +729,23 @@ extern "C" int d3d_topk_rows(const void* logits, int dtype, int N, int64_t V, in
     return err == hipSuccess ? D3D_OK : (int)err;
 }
 
-static size_t lm_slices(int64_t V) { return (size_t)((V + topk::kLmCols - 1) / topk::kLmCols); }
+static size_t lm_slices(int64_t V, int cols) { return (size_t)((V + cols - 1) / cols); }
+
+// The row-streaming kernel: the hidden sizes it is unrolled for, while its
+// slices' candidates fit the merge.
+static bool lm_rows(int H, int64_t V, int k) {
+    return (H == 2048 || H == 4096) && lm_slices(V, topk::kRowCols) * k <= (size_t)topk::kMaxCand;
+}
+
+static size_t lm_bytes(int T, size_t C, int k) {
+    return (((size_t)T * C * k * sizeof(topk::Cand) + 255) & ~(size_t)255) +
+           (((size_t)T * C * sizeof(float2) + 255) & ~(size_t)255);
+}
 
 extern "C" size_t d3d_lmhead_workspace_bytes(int T, int64_t V, int k) {
     if (T < 1 || V < 1 || k < 1) return 0;
-    const size_t C = lm_slices(V);
-    return (((size_t)T * C * k * sizeof(topk::Cand) + 255) & ~(size_t)255) +
-           (((size_t)T * C * sizeof(float2) + 255) & ~(size_t)255);
+    // H is not known here: room for the kernel with the smaller slices.
+    return lm_bytes(T, lm_slices(V, topk::kRowCols), k);
 }
 
 extern "C" int d3d_lmhead_topk(const void* hidden, const void* weight, int T, int H, int64_t V, int k,
@@ -639,8 +758,9 @@ extern "C" int d3d_lmhead_topk(const void* hidden, const void* weight, int T, in
     if (T > 65535 * kLmRows || (int64_t)T > 65535) return D3D_E_SHAPE;  // merge grid: one workgroup per row
     if (!hidden || !weight || !ids_out || !workspace) return D3D_E_NULL;
     if ((uintptr_t)hidden % 16 || (uintptr_t)weight % 16) return D3D_E_UNSUPPORTED;
-    const int C = (int)lm_slices(V);
-    if ((int64_t)C * k > kMaxCand) return D3D_E_SHAPE;
+    if ((int64_t)lm_slices(V, kLmCols) * k > kMaxCand) return D3D_E_SHAPE;
+    const bool rows = lm_rows(H, V, k);
+    const int C = (int)lm_slices(V, rows ? kRowCols : kLmCols);
     if (workspace_bytes < d3d_lmhead_workspace_bytes(T, V, k)) return D3D_E_WORKSPACE;
     LmParams L;
     L.x = static_cast<const uint16_t*>(hidden);
@@ -658,7 +778,12 @@ extern "C" int d3d_lmhead_topk(const void* hidden, const void* weight, int T, in
     // H a multiple of 256: hidden rows staged in LDS; otherwise per-wave loads.
     const bool xlds = H % (32 * kXC) == 0;
     const int kk = k == 1 ? 1 : (k == 2 ? 2 : (k <= 4 ? 4 : 8));
-    switch (kk * 2 + (xlds ? 1 : 0)) {
+    if (rows) {
+        if (kk == 1) launch_lmhead_rows<1>(L, s);
+        else if (kk == 2) launch_lmhead_rows<2>(L, s);
+        else if (kk == 4) launch_lmhead_rows<4>(L, s);
+        else launch_lmhead_rows<8>(L, s);
+    } else switch (kk * 2 + (xlds ? 1 : 0)) {
         case 2: hipLaunchKernelGGL(lmhead_partial_kernel<1>, g1, dim3(rows::NT), 0, s, L); break;
         case 3: hipLaunchKernelGGL(lmhead_partial_xlds_kernel<1>, g1, dim3(rows::NT), 0, s, L); break;
         case 4: hipLaunchKernelGGL(lmhead_partial_kernel<2>, g1, dim3(rows::NT), 0, s, L); break;
