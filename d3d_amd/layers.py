@@ -119,6 +119,28 @@ def project(x: torch.Tensor, weight: torch.Tensor, max_rows: int = ROWS64) -> Pr
     return SplitProduct(parts, splits)
 
 
+def lm_head(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, weight) for bf16 x [..., K] and an LM head [V, K].
+
+    Few rows against many columns stream on d3d_gemm_rows64: up to 32 rows, and
+    up to 64 for K <= 2048.  V = 151,936, us, kernel / hipBLASLt default: 16
+    rows, K = 2048 105 / 211, K = 4096 225 / 264; 64 rows, K = 2048 133 / 156
+    (145 on its tuned solution), K = 4096 263 / 271 (243 tuned, so it stays)."""
+    K, V = x.shape[-1], weight.shape[0]
+    M = x.numel() // K
+    if (not 0 < M <= (ROWS64 if K <= 2048 else 32) or V % 64 or V // 64 < 1024 or K % 128
+            or K // 128 not in _STEPS192 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16
+            or weight.shape[1] != K or not x.is_contiguous() or not weight.is_contiguous() or x.data_ptr() % 16
+            or weight.data_ptr() % 16):
+        return F.linear(x, weight)
+    dev = _lib.require_device(x, weight)
+    y = torch.empty(*x.shape[:-1], V, dtype=torch.bfloat16, device=dev)
+    st = _lib.load().d3d_gemm_rows64(x.data_ptr(), weight.data_ptr(), y.data_ptr(), None, M, V, K, 1,
+                                     _lib.stream_ptr(dev))
+    _lib.check(st, "d3d_gemm_rows64")
+    return y
+
+
 def rows64_silu_ok(H: int, K: int) -> bool:
     """Whether gate_up_silu runs the fused d3d_gemm_rows64_silu_mul for a
     gate-up weight [2H, K] and at most 64 rows: grids of 128 to 512 workgroups

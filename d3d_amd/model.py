@@ -257,7 +257,7 @@ class Qwen3PagedModel(torch.nn.Module):
         return out.reshape(B, Q, s.hidden)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.lm_head)
+        return ly.lm_head(hidden, self.lm_head) if self.rows64_gemm else F.linear(hidden, self.lm_head)
 
 
 # -- page bookkeeping (serving/backend.py:55-76, :123-124) --------------------
