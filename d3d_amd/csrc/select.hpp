@@ -280,6 +280,20 @@ __device__ __forceinline__ float block_incl(float v, float* s, float* tot) {
     return v + off;
 }
 
+// Sum over the workgroup in double: the normalisers of a support, so that their
+// rounding adds nothing to the probabilities' own.
+__device__ __forceinline__ double block_sum_f64(double v, double* s) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    __syncthreads();
+    if ((threadIdx.x & (kWave - 1)) == 0) s[threadIdx.x / kWave] = v;
+    __syncthreads();
+    double t = 0.;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) t += s[w];
+    return t;
+}
+
 // One workgroup per row over its sorted support keys [S]: ids, softmax over
 // the support (max = the first value), the nucleus filter in support order,
 // the draw.  A slot the gather left unwritten (only a NaN logit can leave
@@ -293,10 +307,10 @@ __device__ void support_draw(const uint64_t* k, int S, float top_p, float u, int
         return (kk != ~0ull && z > -INFINITY) ? expf(z - M) : 0.f;
     };
     // Z = sum of the weights, in a fixed order.
-    float part = 0.f;
-    for (int s = threadIdx.x; s < S; s += NTF) part += weight(s);
-    float Z;
-    block_incl(part, s_w, &Z);
+    __shared__ double s_d[kWaves];
+    double sum = 0.;
+    for (int s = threadIdx.x; s < S; s += NTF) sum += (double)weight(s);
+    const float Z = (float)block_sum_f64(sum, s_d);
     // Nucleus filter: entry s > 0 goes when the inclusive probability of
     // entries 0..s-1 exceeds top_p; `keep` is the kept prefix length.
     int keep = S;
@@ -319,13 +333,12 @@ __device__ void support_draw(const uint64_t* k, int S, float top_p, float u, int
     }
     float Zk = Z;
     if (keep < S) {
-        part = 0.f;
-        for (int s = threadIdx.x; s < keep; s += NTF) part += weight(s);
-        block_incl(part, s_w, &Zk);
+        sum = 0.;
+        for (int s = threadIdx.x; s < keep; s += NTF) sum += (double)weight(s);
+        Zk = (float)block_sum_f64(sum, s_d);
     }
     auto prob = [&](int s) { return (s < keep && Zk > 0.f) ? weight(s) / Zk : 0.f; };
-    float tot_p = 0.f;
-    part = 0.f;
+    float tot_p = 0.f, part = 0.f;
     for (int s = threadIdx.x; s < S; s += NTF) {
         const float p = prob(s);
         ids[s] = k[s] == ~0ull ? -1 : (int64_t)(k[s] & ((1ull << kIdBits) - 1));
