@@ -561,11 +561,11 @@ __global__ __launch_bounds__(NT, 2) void lmhead_partial_xlds_kernel(LmParams P) 
 // whole call 166 -> 131.
 constexpr int kRowCols = 128;  // weight rows per workgroup
 
-template <int KK, int MR, int TK, int STEPS>
-__global__ __launch_bounds__(NT) void lmhead_rows_kernel(LmParams P) {
-    constexpr int AR = MR / 16, BC = kRowCols / 4 / 16;  // four waves across the columns
+template <int KK, int MR, int NW, int TK, int STEPS>
+__global__ __launch_bounds__(NW * kWave) void lmhead_rows_kernel(LmParams P) {
+    constexpr int WR = NW / 4, AR = MR / WR / 16, BC = kRowCols / 4 / 16;  // four waves across the columns
     constexpr int STRIDE = kRowCols + 8;                 // bf16 entries per LDS row (16-byte pad)
-    constexpr int TPR = NT / MR, PER = kRowCols / TPR;   // epilogue threads per row, columns each
+    constexpr int TPR = NW * kWave / MR, PER = kRowCols / TPR;  // epilogue threads per row, columns each
     constexpr int LDS = gemm::rows_lds<MR, kRowCols, TK>();
     static_assert(MR * STRIDE * 2 <= LDS, "the logits reuse the tiles");
     __shared__ __attribute__((aligned(16))) char smem[LDS];
@@ -573,7 +573,7 @@ __global__ __launch_bounds__(NT) void lmhead_rows_kernel(LmParams P) {
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int c16 = lane & 15, g4 = lane >> 4;
     gemm::f32x4 acc[AR][BC];
-    gemm::rows_main_loop<MR, kRowCols, 4, 4, TK, 2, STEPS>(
+    gemm::rows_main_loop<MR, kRowCols, NW, 4, TK, 2, STEPS>(
         P.x + (size_t)row0 * P.H, P.w, P.T - row0, P.H, 0, smem,
         [&](int r) { return min(slice * kRowCols + r, P.V - 1); }, acc);
     uint16_t* s_log = reinterpret_cast<uint16_t*>(smem);
@@ -584,7 +584,7 @@ __global__ __launch_bounds__(NT) void lmhead_rows_kernel(LmParams P) {
         for (int b = 0; b < BC; ++b)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                s_log[(16 * a + 4 * g4 + r) * STRIDE + w * (kRowCols / 4) + 16 * b + c16] =
+                s_log[(w / 4 * (MR / WR) + 16 * a + 4 * g4 + r) * STRIDE + w % 4 * (kRowCols / 4) + 16 * b + c16] =
                     f32_to_bf16_bits(acc[a][b][r]);
     __syncthreads();
     // TPR threads per hidden row, PER consecutive slice columns each.
@@ -650,13 +650,20 @@ static void launch_lmhead_rows(const LmParams& L, hipStream_t s) {
     // Up to 16 rows in a 16-row tile (most of the 64-row tile's X loads and
     // MFMAs would be repeats).
     if (L.T <= 16) {
-        if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 16, 128, 16>), dim3(L.C), dim3(NT), 0, s, L);
-        else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 16, 128, 32>), dim3(L.C), dim3(NT), 0, s, L);
+        if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 16, 4, 128, 16>), dim3(L.C), dim3(NT), 0, s, L);
+        else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 16, 4, 128, 32>), dim3(L.C), dim3(NT), 0, s, L);
         return;
     }
-    const dim3 grid(L.C, (L.T + 63) / 64);
-    if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 64, 64, 32>), grid, dim3(NT), 0, s, L);
-    else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 64, 64, 64>), grid, dim3(NT), 0, s, L);
+    // Above 64 rows in 128-row tiles of eight waves: one pass over the weight
+    // per 128 rows (96 rows of 2048 / 4096: 239 / 468 -> 155 / 285 us).
+    if (L.T > 64) {
+        const dim3 grid(L.C, (L.T + 127) / 128);
+        if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 128, 8, 64, 32>), grid, dim3(2 * NT), 0, s, L);
+        else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 128, 8, 64, 64>), grid, dim3(2 * NT), 0, s, L);
+        return;
+    }
+    if (L.H == 2048) hipLaunchKernelGGL((lmhead_rows_kernel<KK, 64, 4, 64, 32>), dim3(L.C), dim3(NT), 0, s, L);
+    else hipLaunchKernelGGL((lmhead_rows_kernel<KK, 64, 4, 64, 64>), dim3(L.C), dim3(NT), 0, s, L);
 }
 
 }  // namespace topk

@@ -25,7 +25,8 @@ def _operands(T, V, H, seed):
 
 
 @pytest.mark.parametrize("H", [2048, 4096])
-@pytest.mark.parametrize("T,V,k", [(1, 129, 1), (16, 5000, 2), (17, 4999, 3), (64, 128, 8), (65, 3001, 5), (128, 40000, 2)])
+@pytest.mark.parametrize("T,V,k", [(1, 129, 1), (16, 5000, 2), (17, 4999, 3), (64, 128, 8), (65, 3001, 5), (128, 40000, 2),
+                                   (129, 2000, 4), (200, 1000, 8)])
 def test_topk_of_the_row_streaming_head(T, V, k, H):
     h, w = _operands(T, V, H, T + V + H)
     ids, vals = lmhead_topk(h, w, k, with_values=True, log_softmax=True)
