@@ -28,9 +28,12 @@
 //       of the X loads, LDS traffic and MFMAs were repeats of the last row.
 //       16 rows: target 12.9 / 8.3 / 19.7 -> 11.5 / 7.5 / 18.7, draft
 //       5.9 / 4.3 / 7.3 -> 5.0 / 3.8 / 6.3.
-//     M <= 64: four waves, TK 64, three stages in flight: target
-//       15.4 / 10.0 / 22.4 -> 15.6 / 9.6 / 22.6, draft 7.3 / 5.6 / 8.9 ->
-//       6.8 / 5.6 / 8.4 against TK 128 and two stages.
+//     M <= 64: four waves; TK 64 and three stages in flight below 2^24
+//       weights, TK 128 and two from there: draft 7.3 / 5.6 / 8.9 with the
+//       latter, 6.8 / 5.6 / 8.4 with the former; target 15.4 / 10.0 / 22.4
+//       and 15.6 / 9.6 / 22.6 alone, but beside the packed prediction on the
+//       other stream the verify forward takes 8.40 ms with TK 128 and 8.84
+//       with TK 64 (engine loop 90.7 against 88.7 steps/s).
 //     M <= 128, 192: eight waves, TK 64, two stages (hipBLASLt before).
 //       128 rows: target 25.7 / 24.4 / 67.4 -> 19.7 / 12.3 / 29.8, draft
 //       14.7 / 11.2 / 17.8 -> 8.6 / 6.9 / 10.9; 192 rows: target
@@ -260,7 +263,8 @@ extern "C" int d3d_gemm_rows64(const void* x, const void* w, void* y, float* par
     const bool done = M <= 16   ? launch_steps<16, 64, 4, 4, 128, 2>(c)
                       : M <= 32 ? launch_steps<32, 64, 4, 4, 128, 2>(c)
                       : wide    ? launch_steps<64, 128, 4, 4, 64, 2>(c)
-                                : launch_steps<64, 64, 4, 4, 64, 3>(c);
+                      : (int64_t)N * K < (1 << 24) ? launch_steps<64, 64, 4, 4, 64, 3>(c)
+                                                   : launch_steps<64, 64, 4, 4, 128, 2>(c);
     if (!done)
         hipLaunchKernelGGL(gemm::gemm_rows64_dma_kernel, dim3(N / gemm::TN, splits), dim3(gemm::NT),
                            gemm::ST * gemm::STAGEB, c.s, c.x, c.w, c.y, parts, M, N, K, K / splits);
