@@ -105,16 +105,6 @@ __device__ __forceinline__ void load_tile(const void* row, int V, int first, int
     constexpr int E = Vec<DT>::E;
     const char* base = static_cast<const char*>(row);
     const bool wide = VEC || V >= E;
-    // A wave wholly inside the row needs no selects (an instruction per entry).
-    if (!__ballot(first + (LT / E - 1) * stride + E > V)) {
-        u32x4 v[LT / E];
-#pragma unroll
-        for (int j = 0; j < LT / E; ++j)
-            v[j] = load16<VEC, STREAM>(base + (size_t)(first + j * stride) * Vec<DT>::bytes);
-#pragma unroll
-        for (int j = 0; j < LT / E; ++j) unpack16<DT>(v[j], x + j * E);
-        return;
-    }
     u32x4 v[LT / E];
     if (wide) {
 #pragma unroll
