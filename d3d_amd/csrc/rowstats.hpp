@@ -104,6 +104,20 @@ template <int DT, bool VEC, bool STREAM, int LT>
 __device__ __forceinline__ void load_tile(const void* row, int V, int first, int stride, float fill, float (&x)[LT]) {
     constexpr int E = Vec<DT>::E;
     const char* base = static_cast<const char*>(row);
+    if constexpr (DT == kF32 && VEC) {
+        // Nothing to unpack, so a branch per vector leaves its load in flight and
+        // saves the clamped form's select per entry (acceptance of 8 requests,
+        // fp32: 38.0 us, 38.6 clamped).
+#pragma unroll
+        for (int j = 0; j < LT / E; ++j) {
+            const int e0 = first + j * stride;
+            u32x4 t;
+            t.x = t.y = t.z = t.w = __float_as_uint(fill);
+            if (e0 + E <= V) t = load16<VEC, STREAM>(base + (size_t)e0 * Vec<DT>::bytes);
+            unpack16<DT>(t, x + j * E);
+        }
+        return;
+    }
     const bool wide = VEC || V >= E;
     u32x4 v[LT / E];
     if (wide) {
