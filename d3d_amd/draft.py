@@ -229,8 +229,9 @@ def sample_with_sparse_probs(logits: torch.Tensor, temperature: float, top_k: in
     probabilities are softmax(z) over the support after the nucleus filter
     (``top_p`` < 1: entry s > 0 is dropped when the mass of entries 0..s-1
     exceeds top_p), and the token is the inverse-CDF draw from them in
-    support order.  Supports of up to 8 entries take the top-k rounds and one
-    wave per row; wider ones the sorted-support path.
+    support order.  Supports of up to 8 entries, and up to 64 of rows the
+    sorted-support path does not take (V > 2^18), take the top-k kernels and one
+    wave per row; the others the sorted-support path.
     """
     dev = _lib.require_device(logits)
     if not temperature > 1e-5:
@@ -248,7 +249,7 @@ def sample_with_sparse_probs(logits: torch.Tensor, temperature: float, top_k: in
     u = _uniforms(lg.shape[:-1], dev, uniforms, generator)
     tok = torch.empty(lg.shape[:-1], dtype=torch.int64, device=dev)
     probs = torch.empty(*lg.shape[:-1], S, dtype=torch.float32, device=dev)
-    if S > 8:
+    if S > 64 or (S > 8 and V <= _lib.FILTER_MAX_V):
         ids = torch.empty(*lg.shape[:-1], S, dtype=torch.int64, device=dev)
         lib = _lib.load()
         nbytes = lib.d3d_support_workspace_bytes(max(N, 1), S)
