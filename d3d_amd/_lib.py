@@ -24,6 +24,8 @@ D3D_CONF_MAX_SOFTMAX = 0
 D3D_CONF_ONE_HOT = 1
 FILTER_MAX_K = 4096  # top_k and vocabulary d3d_filter_rows takes
 FILTER_MAX_V = 1 << 18
+TOPK_MAX_K = 64  # k and candidates per row (k for each 4096 entries) d3d_topk_rows takes
+TOPK_MAX_CANDIDATES = 8192
 D3D_TOKEN_EMPTY_DISTRIBUTION = -1
 D3D_TOKEN_BAD_DRAFT = -2
 D3D_TOKEN_TIMEOUT = -3
