@@ -179,9 +179,13 @@ __global__ __launch_bounds__(NT) void topk_chunk_kernel(Params P) {
     }
 }
 
-// NTM threads: 1024 for more than 1,024 candidates (the LM head's 1,187 slices),
-// whose loads and rounds a 256-thread workgroup walks nine deep: the LM head's
-// whole call at 64 rows, k = 2 136.8 -> 133.6 us, k = 6 192.8 -> 173.8.
+// NTM threads: 1024 for more than 1,024 slices (the LM head's 1,187) or more
+// than 2,048 candidates, whose loads and rounds a 256-thread workgroup walks
+// nine deep: the LM head's whole call at 64 rows, k = 2 136.8 -> 133.6 us, k = 6
+// 192.8 -> 173.8.  A round's argmax costs more over sixteen waves, so several
+// rounds over fewer candidates stay with 256 threads (one bf16 row of 262,145,
+// 256 / 1024 threads: k = 16, 1,040 candidates, 36.4 / 42.8 us; k = 30, 1,950,
+// 79.7 / 80.0; k = 40, 2,600, 122.6 / 108.1).
 template <int NTM>
 __global__ __launch_bounds__(NTM) void topk_merge_kernel(Params P) {
     const int n = blockIdx.x;
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(NTM) void topk_merge_kernel(Params P) {
 }
 
 static void launch_merge(const Params& P, int rows, hipStream_t s) {
-    if (P.C * P.k > 1024)
+    if (P.C > 1024 || P.C * P.k > 2048)
         hipLaunchKernelGGL(topk_merge_kernel<1024>, dim3(rows), dim3(1024), 0, s, P);
     else
         hipLaunchKernelGGL(topk_merge_kernel<NT>, dim3(rows), dim3(NT), 0, s, P);

@@ -69,3 +69,12 @@ def test_a_wider_top_k_or_a_nucleus_takes_the_general_filter():
         # a cut within an fp32 sum's rounding of p may fall one entry off
         assert bool(((probs > 0).sum(-1) - (q > 0).sum(-1)).abs().max() <= 1)
         assert torch.allclose(probs.sum(-1), torch.ones(N), rtol=1e-4)
+
+
+@pytest.mark.parametrize("k", [16, 31, 32, 64])  # 65 chunks: 1,040, 2,015, 2,080 and 4,160 candidates in the merge
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_top_k_on_both_sides_of_the_wide_merge(k, dtype):
+    x = _rows(2, dtype, k)
+    ids, vals = dr.topk_tokens(x.to(DEV), k, with_values=True)
+    order = x.float().sort(dim=-1, descending=True, stable=True)
+    assert torch.equal(ids.cpu(), order.indices[:, :k]) and torch.equal(vals.cpu(), order.values[:, :k])
