@@ -208,13 +208,60 @@ __device__ __forceinline__ uint64_t support_key(float z, int e) {
     return ((uint64_t)(~key_of(z)) << kIdBits) | (uint64_t)e;
 }
 
-// Every entry z >= z_t of the row's passing groups into list (any order);
-// returns their number, which may exceed kMaxSel (then list is incomplete),
-// or -1 when more groups pass than fit.  z_t is at most the k-th largest z.
+// Notes group i as passing (any order).
+__device__ __forceinline__ void list_group(int i, bool hit, uint16_t* groups, SelScratch& sc) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint64_t bal = __ballot(hit);
+    if (bal) {
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(&sc.s.n_groups, (uint32_t)__popcll(bal));
+        base = (uint32_t)__shfl((int)base, 0, kWave) + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
+        if (hit && base < (uint32_t)kMaxGroups) groups[base] = (uint16_t)i;
+    }
+}
+
+// The passing groups' entries with z > lo (none has x < x_lo) into list;
+// returns their number, or -1 when they or the groups do not fit.
+template <int DT, bool VEC>
+__device__ __forceinline__ int gather_groups(const SelParams& P, const void* row, float x_lo, float lo, bool unit,
+                                             uint64_t* list, const uint16_t* groups, SelScratch& sc) {
+    constexpr int E = rows::Vec<DT>::E;
+    __syncthreads();
+    const int ng = (int)sc.s.n_groups;
+    if (ng > kMaxGroups) return -1;
+    constexpr int PP = kGroup / E;  // 16-byte pieces of a group
+    for (int p = threadIdx.x; p < ng * PP; p += NTF) {
+        const int gi = groups[p / PP];
+        const int e0 = (gi / NT) * kChunk + (gi % NT) * E + (p % PP) * NT * E;
+        float x[E];
+        rows::load_tile<DT, VEC, false, E>(row, P.V, e0, 0, -INFINITY, x);
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            if (e0 + q < P.V && !(x[q] < x_lo)) {
+                const float z = unit ? x[q] : x[q] / P.T;
+                if (z > lo) {
+                    const uint32_t slot = atomicAdd(&sc.s.n_cand, 1u);
+                    if (slot < (uint32_t)kMaxSel) list[slot] = support_key(z, e0 + q);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int m = (int)sc.s.n_cand;
+    return m <= kMaxSel ? m : -1;
+}
+
+// The row's entries z >= z_t into list (any order), z_t at most its k-th
+// largest z; returns their number, or -1 when they do not fit.  When they do
+// not, or z_t = -inf, only the entries above z_t: fewer than k of those leave
+// the others of the k largest to append_ties(z_t).  That is a row with a long
+// run of equal values at its k-th largest, above all a masked one (-inf or a
+// dtype's lowest value): in the general selection's passes every count of such
+// a run hits one bin.  64 bf16 rows of 151,936, 20 entries not masked, us,
+// general / this: top-64 592 / 17, support of 64 600 / 24, top-50 draw 697 / 22.
 template <int DT, bool VEC>
 __device__ int collect(const SelParams& P, const void* row, const float* gmax, int k, bool unit, uint64_t* list,
-                       uint16_t* groups, SelScratch& sc) {
-    constexpr int E = rows::Vec<DT>::E;
+                       uint16_t* groups, SelScratch& sc, float& z_t) {
     const int G = P.C * NT, lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     float g[kRegKeys];
     uint32_t key[kRegKeys];
@@ -318,46 +365,61 @@ __device__ int collect(const SelParams& P, const void* row, const float* gmax, i
         }
     }
     __syncthreads();
+    // A negative bf16 maximum's key ends in ones.
+    if (DT == kBF16 && t < 0x80000000u) t |= 0xffffu;
     const float x_t = t > 0x007fffffu ? float_of(t) : -INFINITY;  // 0x007fffff: the key of -inf
-    const float z_t = unit ? x_t : x_t / P.T;
+    z_t = unit ? x_t : x_t / P.T;
     // Nothing below x_lo scales to z_t: equal quotients lie within a few ulp.
     const float x_lo = x_t - fabsf(x_t) * 0x1p-20f;
+    // Entries above lo are taken.
+    const float lo = z_t == -INFINITY ? z_t : float_below(z_t);
 #pragma unroll
     for (int j = 0; j < kRegKeys; ++j) {
         if (j >= J) break;
         const int i = j * NTF + (int)threadIdx.x;
-        bool hit = i < G && !(g[j] < x_lo);
-        if (hit) hit = (unit ? g[j] : g[j] / P.T) >= z_t;
+        list_group(i, i < G && !(g[j] < x_lo) && (unit ? g[j] : g[j] / P.T) > lo, groups, sc);
+    }
+    int m = gather_groups<DT, VEC>(P, row, x_lo, lo, unit, list, groups, sc);
+    if (m >= 0 || lo == z_t) return m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sc.s.n_groups = 0;
+        sc.s.n_cand = 0;
+    }
+    __syncthreads();
+    for (int j = 0; j < J; ++j) {
+        const int i = j * NTF + (int)threadIdx.x;
+        const float x = gmax[min(i, G - 1)];
+        list_group(i, i < G && !(x < x_lo) && (unit ? x : x / P.T) > z_t, groups, sc);
+    }
+    return gather_groups<DT, VEC>(P, row, x_lo, z_t, unit, list, groups, sc);
+}
+
+// Appends the row's first entries (by id) with z == v to the m entries of list
+// until it holds k, and returns the count; a masked row has enough of them in
+// its first thousand.
+template <int DT>
+__device__ int append_ties(const SelParams& P, const void* row, float v, int m, int k, bool unit, uint64_t* list,
+                           SelScratch& sc) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    for (int base = 0, par = 0; base < P.V && m < k; base += NTF, par ^= 1) {
+        const int e = base + (int)threadIdx.x;
+        const bool hit = e < P.V && scaled<DT>(row, e, P.T, unit) == v;
         const uint64_t bal = __ballot(hit);
-        if (bal) {
-            uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(&sc.s.n_groups, (uint32_t)__popcll(bal));
-            base = (uint32_t)__shfl((int)base, 0, kWave) + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
-            if (hit && base < (uint32_t)kMaxGroups) groups[base] = (uint16_t)i;
-        }
-    }
-    __syncthreads();
-    const int ng = (int)sc.s.n_groups;
-    if (ng > kMaxGroups) return -1;
-    constexpr int PP = kGroup / E;  // 16-byte pieces of a group
-    for (int p = threadIdx.x; p < ng * PP; p += NTF) {
-        const int gi = groups[p / PP];
-        const int e0 = (gi / NT) * kChunk + (gi % NT) * E + (p % PP) * NT * E;
-        float x[E];
-        rows::load_tile<DT, VEC, false, E>(row, P.V, e0, 0, -INFINITY, x);
+        uint32_t* slot = sc.s.cnt[par];
+        if (lane == 0) slot[w] = (uint32_t)__popcll(bal);
+        __syncthreads();
+        int at = m + __popcll(bal & ((1ull << lane) - 1)), total = 0;
 #pragma unroll
-        for (int q = 0; q < E; ++q) {
-            if (e0 + q < P.V && !(x[q] < x_lo)) {
-                const float z = unit ? x[q] : x[q] / P.T;
-                if (z >= z_t) {
-                    const uint32_t slot = atomicAdd(&sc.s.n_cand, 1u);
-                    if (slot < (uint32_t)kMaxSel) list[slot] = support_key(z, e0 + q);
-                }
-            }
+        for (int q = 0; q < kWaves; ++q) {
+            at += q < w ? (int)slot[q] : 0;
+            total += (int)slot[q];
         }
+        if (hit && at < k) list[at] = support_key(v, e);
+        m = min(m + total, k);
     }
     __syncthreads();
-    return (int)sc.s.n_cand;
+    return m;
 }
 
 // Exactly the k largest entries (ties by id) of a row collect() could not
@@ -567,11 +629,21 @@ __global__ __launch_bounds__(NTF) void select_kernel(SelParams P) {
     const int n = blockIdx.x, k = P.k;
     const bool unit = P.T == 1.0f;
     const void* row = rows::row_ptr<DT>(P.logits, n, P.V);
-    int m = collect<DT, VEC>(P, row, P.gmax + (size_t)n * P.C * NT, k, unit, list, groups, sc);
-    const bool fits = m >= 0 && m <= kMaxSel;
+    float tie;
+    int m = collect<DT, VEC>(P, row, P.gmax + (size_t)n * P.C * NT, k, unit, list, groups, sc, tie);
+    const bool fits = m >= 0, tied = fits && m < k;
+    if (tied) m = append_ties<DT>(P, row, tie, m, k, unit, list, sc);
     if constexpr (M == kFilter) {
         // NaN entries may be among the k largest only if fewer others exist.
-        if (!fits || m < k) {
+        bool general = !fits || m < k;
+        if (tied && !general) {
+            // Every entry at the tie is kept; the list holds the first few of
+            // them, which is enough if they weigh nothing.
+            float mx = -INFINITY;
+            for (int i = threadIdx.x; i < m; i += NTF) mx = fmaxf(mx, key_value(list[i]));
+            general = weight_fx(tie, row_max(mx, sc)) != 0;
+        }
+        if (general) {
             const float* gm = P.gmax + (size_t)n * P.C * NT;
             float mx = -INFINITY;
             for (int i = threadIdx.x; i < P.C * NT; i += NTF) mx = fmaxf(mx, gm[i]);
@@ -617,7 +689,9 @@ __global__ __launch_bounds__(NTF) void select_kernel(SelParams P) {
         }
         draw_from_segments<DT, 1>(P, row, n, P.C, mx, zf, lim, Scale(P.T), sc);
     } else if constexpr (M == kSupport) {
-        if (!fits || (m < k && k < P.V)) m = collect_general<DT>(P, row, k, unit, list, sc);
+        // A support short of k entries (NaN elsewhere): up to 64 the slots stay
+        // empty, as with the top-k kernels, wider ones list NaN entries by id.
+        if (!fits || (m < k && k > 64 && k < P.V)) m = collect_general<DT>(P, row, k, unit, list, sc);
         pad_and_sort(list, m, k, sc.s.rank);
         support_draw(list, k, P.top_p, P.u[n], P.tok + n, P.ids + (size_t)n * k, P.probs + (size_t)n * k,
                      P.tok_prob ? P.tok_prob + n : nullptr, sc.s.f, sc.s.i);

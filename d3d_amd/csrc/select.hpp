@@ -43,6 +43,12 @@ __device__ __forceinline__ float float_of(uint32_t k) {
     return __uint_as_float(u);
 }
 
+// The largest float below z > -inf (-0 is read as +0).
+__device__ __forceinline__ float float_below(float z) {
+    const uint32_t k = key_of(z) - 1;
+    return float_of(k == 0x7fffffffu ? k - 1 : k);  // 0x7fffffff: the key -0 would have
+}
+
 template <int DT>
 __device__ __forceinline__ float scaled(const void* row, int e, float T, bool unit) {
     const float x = rows::load_one<DT>(row, e);
