@@ -369,8 +369,10 @@ __device__ int collect(const SelParams& P, const void* row, const float* gmax, i
     if (DT == kBF16 && t < 0x80000000u) t |= 0xffffu;
     const float x_t = t > 0x007fffffu ? float_of(t) : -INFINITY;  // 0x007fffff: the key of -inf
     z_t = unit ? x_t : x_t / P.T;
-    // Nothing below x_lo scales to z_t: equal quotients lie within a few ulp.
-    const float x_lo = x_t - fabsf(x_t) * 0x1p-20f;
+    // Nothing below x_lo scales to z_t: numerators of equal quotients lie within
+    // T times the quotient's ulp, a few ulp of x_t, or T 2^-149 where the
+    // quotient is denormal.
+    const float x_lo = x_t - fmaxf(fabsf(x_t) * 0x1p-20f, P.T * 0x1p-147f);
     // Entries above lo are taken.
     const float lo = z_t == -INFINITY ? z_t : float_below(z_t);
 #pragma unroll

@@ -165,3 +165,26 @@ def test_scaling_that_overflows_counts_as_minus_infinity():
     tok, sid, probs = dr.sample_with_sparse_probs(x.to(DEV), T, k, uniforms=torch.zeros(1, device=DEV))
     assert sid[0].tolist() == [5001, 5003, 5002, 5000] + list(range(8))
     assert int(tok[0]) == 5001 and bool((probs[0, 4:] == 0).all())
+
+
+@pytest.mark.parametrize("unit,T", [(2.0 ** -149, 1.7), (2.0 ** -149, 40.0), (2.0 ** -120, 3e8), (2.0 ** -30, 3.3e38)])
+@pytest.mark.parametrize("k", [20, 300])
+def test_denormal_quotients_tie(unit, T, k):
+    """Small multiples of a unit whose quotients by T are a few denormals (or zeros), so different entries tie."""
+    V, N = 20000, 4
+    g = torch.Generator().manual_seed(k)
+    x = (torch.randint(-400, 401, (N, V), generator=g).double() * unit).float()
+    x[1:] = x[1:] * (torch.rand(N - 1, V, generator=g) < 0.05)
+    z = (x.double() / float(np.float32(T))).float()  # the double quotient rounds once: denormals have few bits
+    u = torch.rand(N, generator=g)
+    tok, sid, probs = dr.sample_with_sparse_probs(x.to(DEV), T, k, uniforms=u.to(DEV))
+    np.testing.assert_array_equal(sid.cpu().numpy(), _sorted_ids(z, k))
+    zf, lim = dr._filters(x.to(DEV), T, k, 1.0, True)
+    kth = z.sort(dim=-1, descending=True).values[:, k - 1]
+    assert torch.equal(zf.cpu(), kth) and bool((lim.cpu() == 2 ** 31 - 1).all())
+    # Every kept entry weighs the same (exp(0)): the draw is the floor(u n)-th kept id.
+    tok, prob = (t.cpu() for t in dr.sample_with_prob(x.to(DEV), T, k, uniforms=u.to(DEV)))
+    for n in range(N):
+        kept = torch.nonzero(z[n] >= kth[n])[:, 0]
+        at = int(float(u[n]) * len(kept))
+        assert int(tok[n]) == int(kept[at]) and abs(float(prob[n]) * len(kept) - 1) < 1e-6
