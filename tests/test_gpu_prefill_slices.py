@@ -37,3 +37,16 @@ def test_wide_slices_equal_narrow_ones(lens):
     assert (h.float() - h1.float()).norm() <= 0.02 * h1.float().norm()
     for a, b in zip(kv, kv1):
         assert a.shape == b.shape and (a.float() - b.float()).norm() <= 0.02 * b.float().norm()
+
+
+@pytest.mark.parametrize("lens,block", [((14,) * 300, 16), ((2049, 2100), 32)])
+def test_rows_that_go_through_the_model(lens, block, monkeypatch):
+    """Many short prompts keep the default slices, a caller's own block stays as it is."""
+    model = Qwen3PagedModel(TINY, DEV, draft=False, seed=3, init_std=0.05)
+    shapes = []
+    forward = model.forward
+    monkeypatch.setattr(model, "forward", lambda ids, *a, **kw: shapes.append(tuple(ids.shape)) or forward(ids, *a, **kw))
+    kv = PagedKV(TINY, 400, 16, DEV)
+    with torch.inference_mode():
+        prefill(model, kv, [Sequence(i, [1] * n) for i, n in enumerate(lens)], "t", block=block)
+    assert shapes == [(sum(-(-n // block) for n in lens), block)]
