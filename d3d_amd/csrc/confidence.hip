@@ -65,8 +65,8 @@ __global__ __launch_bounds__(NT) void conf_stats_kernel(Params P) {
     const int first = c * kChunk + threadIdx.x * E;
     float x[L];
     load_tile<DT, VEC, true, L>(row, P.V, first, NT * E, fill_value<kLogits>(), x);
-    const RowStat st = P.T == 1.0f ? chunk_stats<DT, kLogits, true, true>(x, first, P.T, true, rf, ri)
-                                   : chunk_stats<DT, kLogits, false, true>(x, first, P.T, true, rf, ri);
+    const RowStat st = P.T == 1.0f ? chunk_stats<DT, kLogits, true>(x, first, P.T, true, rf, ri)
+                                   : chunk_stats<DT, kLogits, false>(x, first, P.T, true, rf, ri);
     if (threadIdx.x == 0) P.stats[((size_t)b * P.Q + i) * P.C + c] = st;
 }
 

@@ -268,23 +268,7 @@ __device__ __forceinline__ int block_min_int(int v, int* scratch) {
     return r;
 }
 
-// exp(d) for d <= 0 (0 below -200, NaN for NaN) to about one unit in the last
-// place: 2^t on the transcendental unit for t = d log2 e rounded, times
-// 1 + ln 2 * (the rounding's error, exact by a multiply-add, and the rest of
-// log2 e).  10 instructions' worth against 17 of expf, which the row passes,
-// bound by their VALU work, spend half of their time on.
-__device__ __forceinline__ float exp_nonpos(float d) {
-    constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596299e-8f, kLn2 = 0.693147181f;
-    d = d < -200.f ? -200.f : d;
-    const float t = d * kLog2e;
-    const float r = __builtin_fmaf(d, kLog2eRest, __builtin_fmaf(d, kLog2e, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    return __builtin_fmaf(e, r * kLn2, e);
-}
-
-// FAST_EXP: exp_nonpos in place of expf.  Acceptance keeps expf: its decisions
-// and tokens are pinned to those sums' bits.
-template <int DT, Mode M, bool UNIT_T, bool FAST_EXP = false>
+template <int DT, Mode M, bool UNIT_T>
 __device__ __forceinline__ RowStat chunk_stats(const float (&x)[L], int first, float T, bool want_arg,
                                                float* rf, int* ri) {
     constexpr int E = Vec<DT>::E;
@@ -326,7 +310,7 @@ __device__ __forceinline__ RowStat chunk_stats(const float (&x)[L], int first, f
             for (int l = 0; l < L; ++l) z[l] = x[l];
             if constexpr (!UNIT_T) Scale(T).tile(z);
 #pragma unroll
-            for (int l = 0; l < L; ++l) s += FAST_EXP ? exp_nonpos(z[l] - m) : expf(z[l] - m);
+            for (int l = 0; l < L; ++l) s += expf(z[l] - m);
         }
         st.m = m;
         st.s = block_sum<NT>(s, rf);

@@ -97,7 +97,7 @@ __global__ __launch_bounds__(NT) void sample_stats_kernel(Params P) {
         apply_floor<UNIT_T>(P, n, x);
         apply_filter<DT, UNIT_T>(P, n, first, NT * E, x);
     }
-    const RowStat st = chunk_stats<DT, M, UNIT_T, true>(x, first, P.T, M == kGreedy, rf, ri);
+    const RowStat st = chunk_stats<DT, M, UNIT_T>(x, first, P.T, M == kGreedy, rf, ri);
     if (threadIdx.x == 0) P.stats[(size_t)n * P.C + c] = st;
 }
 

@@ -139,3 +139,22 @@ def test_support_and_topk_match_a_stable_sort(kind, V, S, dtype):
         top, vals = dr.topk_tokens(x, S, with_values=True)
         np.testing.assert_array_equal(top.cpu().numpy(), _sorted_ids(x, 1.0, S))
         assert torch.equal(vals, x.float().gather(1, top))
+
+
+def test_masses_are_as_exact_as_the_exponential_allows():
+    """Rows of one 0, n entries of one d and a filtered one, the 0 drawn: its
+    probability is 1 / W, W = 1 + n e^d.  In units of 2^-20 of W's value (the
+    spacing at [8, 16)), rms: W's rounding 0.289; the quotient's, 2^-27 of p
+    against p W^-1 2^-20, 0.289 W^2 / 128, 0.38 over these W; n times e^d's own
+    error, 62 / 64 of a unit for each 2^-26 of e^d: 0.29 for the 0.30 of an
+    argument-reduced exponential.  Together 0.56, and 0.62 with an e^d of 0.40."""
+    N, n, V = 65535, 62, 64
+    d = torch.linspace(-2.07, -1.39, N).float()  # e^d in [1/8, 1/4), the sum in [8, 16.5)
+    x = d[:, None].repeat(1, V)
+    x[:, 0] = 0.0
+    x[:, V - 1] = -50.0
+    tok, prob = dr.sample_with_prob(x.to(DEV), 1.0, V - 1, uniforms=torch.zeros(N, device=DEV))
+    assert bool((tok == 0).all())
+    exact = 1.0 / (1.0 + n * d.double().exp())
+    err = (prob.cpu().double() / exact - 1) / (exact * 2.0 ** -20)
+    assert float(err.square().mean().sqrt()) < 0.59
