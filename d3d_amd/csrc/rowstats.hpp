@@ -5,6 +5,7 @@
 #pragma once
 
 #include "d3d_common.hpp"
+#include "scalar_math.hpp"
 
 #include <limits.h>
 
@@ -141,43 +142,40 @@ __device__ __forceinline__ void load_tile(const void* row, int V, int first, int
     }
 }
 
-// x / T, correctly rounded as the division is, in three multiply-adds: with
-// inv = 1 / T correctly rounded, q = x * inv is within one unit of the
-// quotient, r = x - q * T is exact, and q + r * inv rounds to x / T
-// (Markstein's theorem; it excludes a T whose mantissa is all ones).  Entries
-// whose intermediate values could leave the normal range, zeros, infinities
-// and NaN take the division.  The row passes are VALU-bound (the division is
-// about 10 of some 40 instructions per entry): sparse acceptance's pass over
-// 128 bf16 rows of 151,936 at T = 0.7 22.9 -> 20.0 us, the same bits.
+// x / T, rounded as the division rounds it, by multiply-adds (Quotient).
+// Entries whose intermediate values could leave the normal range, zeros,
+// infinities and NaN take the division.  The row passes are VALU-bound (the
+// division is about 10 of some 40 instructions per entry): sparse acceptance's
+// pass over 128 bf16 rows of 151,936 at T = 0.7 22.9 -> 20.0 us, the same bits.
 struct Scale {
-    float T, inv;
+    Quotient q;
     bool unit, fast;
     __device__ __forceinline__ explicit Scale(float t)
-        : T(t), inv(1.0f / t), unit(t == 1.0f),
+        : q(t), unit(t == 1.0f),
           fast(t > 0x1p-20f && t < 0x1p40f && (__float_as_uint(t) & 0x7fffffu) != 0x7fffffu) {}
     // x[] <- x[] / T.  The wave takes the division if any entry needs it: a
     // branch per entry would leave no two entries' chains overlapping.
     template <int LT>
     __device__ __forceinline__ void tile(float (&x)[LT]) const {
         if (unit) return;
-        if (fast) {
-            float z[LT];
-            bool odd = false;
+        if (fast && (q.direct ? by_quotient<true>(x) : by_quotient<false>(x))) return;
 #pragma unroll
-            for (int l = 0; l < LT; ++l) {
-                const float q = x[l] * inv;
-                z[l] = __builtin_fmaf(__builtin_fmaf(-q, T, x[l]), inv, q);
-                // |x| outside [2^-60, 2^60)
-                odd |= (__float_as_uint(x[l]) & 0x7fffffffu) - 0x21800000u >= 0x3c000000u;
-            }
-            if (!__ballot(odd)) {
+        for (int l = 0; l < LT; ++l) x[l] = x[l] / q.T;
+    }
+    template <bool DIRECT, int LT>
+    __device__ __forceinline__ bool by_quotient(float (&x)[LT]) const {
+        float z[LT];
+        bool odd = false;
 #pragma unroll
-                for (int l = 0; l < LT; ++l) x[l] = z[l];
-                return;
-            }
+        for (int l = 0; l < LT; ++l) {
+            z[l] = q.of<DIRECT>(x[l]);
+            // |x| outside [2^-60, 2^60)
+            odd |= (__float_as_uint(x[l]) & 0x7fffffffu) - 0x21800000u >= 0x3c000000u;
         }
+        if (__ballot(odd)) return false;
 #pragma unroll
-        for (int l = 0; l < LT; ++l) x[l] = x[l] / T;
+        for (int l = 0; l < LT; ++l) x[l] = z[l];
+        return true;
     }
 };
 

@@ -6,7 +6,6 @@
 
 #include "d3d_common.hpp"
 #include "rowstats.hpp"
-#include "scalar_math.hpp"
 #include "../../include/d3d_hip.h"
 
 #include <limits.h>

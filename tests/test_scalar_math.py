@@ -61,3 +61,47 @@ def test_reduced_exponential(tmp_path):
     # twice more: 1.0 and 0.41.
     assert worst < 0.7 and max(rms) < 0.31
     assert one and small and nan
+
+
+QUOTIENT = r"""
+#include <cmath>
+#include <cstdint>
+#include <cstdio>
+#include <cstring>
+#include "scalar_math.hpp"
+template <bool DIRECT>
+static void sweep(float T, const d3d::Quotient& q) {
+    double off = 0;
+    long bad = 0;
+    for (uint32_t m = 0; m < (1u << 23); ++m) {
+        const uint32_t u = 0x3f800000u | m;
+        float x;
+        std::memcpy(&x, &u, 4);
+        const double exact = (double)x / (double)T;
+        const double unit = std::ldexp(1.0, std::ilogb(exact) - 23);
+        off = std::fmax(off, std::fabs(q.first<DIRECT>(x) - exact) / unit);
+        bad += q.of<DIRECT>(x) != x / T;
+    }
+    std::printf("%.6f %ld ", off, bad);
+}
+int main(int argc, char** argv) {
+    const float ts[] = {TEMPERATURES};
+    for (float T : ts) {
+        const d3d::Quotient q(T);
+        if (q.direct) sweep<true>(T, q);
+        sweep<false>(T, q);
+    }
+}
+"""
+
+
+@pytest.mark.parametrize("ts", ["0.7f, 0.8f, 1.3f, 0.9f", "1.7f, 1.95f, 0.95f, 0.487f",
+                                "0x1.fffff8p0f, 0x1.fffffcp0f, 0x1.000002p0f, 0x1.000004p0f"])
+def test_quotients_round_as_the_division(ts, tmp_path):
+    """Every mantissa of x at temperatures of either kind and next to powers of
+    two (the worst 1 / T): q within the unit that the theorem asks for, and the
+    division's bits.  q = x * inv alone is up to 1.5 units off."""
+    out = _run(tmp_path, QUOTIENT.replace("TEMPERATURES", ts))
+    assert len(out) >= 8
+    for off, bad in zip(out[::2], out[1::2]):
+        assert float(off) <= 1.0 and int(bad) == 0
