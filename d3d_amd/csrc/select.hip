@@ -24,8 +24,9 @@
 // top_p * S are gathered;
 // (4) one workgroup per row narrows them down the same way and places the cut.
 // All masses are 64-bit integers, so the cut does not depend on the order of
-// the sums and equals the general filter's.  A draw uses the same integers:
-// the parts' masses, then one part's entries in id order.
+// the sums and equals the general filter's.  A draw uses integers too (the same
+// ones, or of a finer unit where few entries are kept): the parts' masses, then
+// one part's entries in id order.
 //
 // Measured, 64 bf16 rows of 151,936 (19.4 MB, 4 us at the copy rate): sorted
 // top-64 with its draw 236 -> 21.6 us (k rounds of argmaxes over every chunk
@@ -505,10 +506,15 @@ __device__ int first_crossing(const uint64_t* list, int m, float M, uint64_t A, 
     return r;
 }
 
+// Units of a draw's weights, as fine as their sum allows (at most 2^64): a
+// top-k's kept entries in LDS, a whole row.
+constexpr int kListBits = 50, kRowBits = 45;
+static_assert(kMaxSel <= 1 << (63 - kListBits) && kMaxV <= 1 << (63 - kRowBits), "sum of the weights");
+
 // Inverse-CDF draw over the kept entries (zf, lim) in id order, from the
-// masses of the row's `segs` segments of SPAN chunks in sc.s.mass: first t
-// with C_t > u * W, else the last with mass.
-template <int DT, int SPAN>
+// masses of the row's `segs` segments of SPAN chunks in sc.s.mass, sums of
+// draw_fx<BITS>: first t with C_t > u * W, else the last with mass.
+template <int DT, int SPAN, int BITS>
 __device__ void draw_from_segments(const SelParams& P, const void* row, int n, int segs, float M, float zf, int lim,
                                    const Scale& scale, SelScratch& sc) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -524,7 +530,7 @@ __device__ void draw_from_segments(const SelParams& P, const void* row, int n, i
             sc.s.i[0] = c;
             // Mass still to pass inside the segment; all of it when nothing crosses.
             sc.s.base = over ? target - (incl - m) : ~0ull;
-            sc.s.fx = (float)((double)W / kFix);
+            sc.s.fx = (float)((double)W / (double)(1ull << BITS));
         }
     }
     __syncthreads();
@@ -548,7 +554,7 @@ __device__ void draw_from_segments(const SelParams& P, const void* row, int n, i
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
         const bool kept = e0 + q < P.V && (z[q] > zf || (z[q] == zf && e0 + q <= lim));
-        wt[q] = kept ? weight_fx(z[q], M) : 0;
+        wt[q] = kept ? draw_fx<BITS>(z[q], M) : 0;
         sum += wt[q];
     }
     uint64_t tot;
@@ -605,13 +611,13 @@ __device__ void filter_row_general(const SelParams& P, const void* row, int n, f
         uint64_t w = 0;
         if (e < P.V) {
             const float z = scaled<DT>(row, e, P.T, unit);
-            if (z > zf || (z == zf && e <= lim)) w = weight_fx(z, M);
+            if (z > zf || (z == zf && e <= lim)) w = draw_fx<kRowBits>(z, M);
         }
         const uint64_t s = wave_incl_u64(w, threadIdx.x & (kWave - 1));
         if ((threadIdx.x & (kWave - 1)) == kWave - 1 && s)
             atomicAdd((unsigned long long*)&sc.s.mass[e / kChunk], (unsigned long long)s);
     }
-    draw_from_segments<DT, 1>(P, row, n, P.C, M, zf, lim, Scale(P.T), sc);
+    draw_from_segments<DT, 1, kRowBits>(P, row, n, P.C, M, zf, lim, Scale(P.T), sc);
 }
 
 // Row maximum of the scaled logits (the caller's value is per thread).
@@ -643,7 +649,7 @@ __global__ __launch_bounds__(NTF) void select_kernel(SelParams P) {
             // them, which is enough if they weigh nothing.
             float mx = -INFINITY;
             for (int i = threadIdx.x; i < m; i += NTF) mx = fmaxf(mx, key_value(list[i]));
-            general = weight_fx(tie, row_max(mx, sc)) != 0;
+            general = draw_fx<kMassBits>(tie, row_max(mx, sc)) != 0;
         }
         if (general) {
             const float* gm = P.gmax + (size_t)n * P.C * NT;
@@ -685,11 +691,11 @@ __global__ __launch_bounds__(NTF) void select_kernel(SelParams P) {
         for (int c = threadIdx.x; c < kMaxChunks; c += NTF) sc.s.mass[c] = 0;
         __syncthreads();
         for (int i = threadIdx.x; i < keep; i += NTF) {
-            const uint64_t w = weight_fx(key_value(list[i]), mx);
+            const uint64_t w = draw_fx<kListBits>(key_value(list[i]), mx);
             const int c = (int)(list[i] & ((1ull << kIdBits) - 1)) / kChunk;
             if (w) atomicAdd((unsigned long long*)&sc.s.mass[c], (unsigned long long)w);
         }
-        draw_from_segments<DT, 1>(P, row, n, P.C, mx, zf, lim, Scale(P.T), sc);
+        draw_from_segments<DT, 1, kListBits>(P, row, n, P.C, mx, zf, lim, Scale(P.T), sc);
     } else if constexpr (M == kSupport) {
         // A support short of k entries (NaN elsewhere): up to 64 the slots stay
         // empty, as with the top-k kernels, wider ones list NaN entries by id.
@@ -1014,10 +1020,12 @@ __global__ __launch_bounds__(NTF) void nucleus_finish_kernel(SelParams P) {
         const int c = (int)(key & ((1ull << kIdBits) - 1)) / (kChunk * P.span);
         if (w) atomicAdd((unsigned long long*)&sc.s.mass[c], (unsigned long long)w);
     }
+    // The cut's entry weighs at least one unit, so every kept one does, and the
+    // masses are draw_fx's.
     if (P.span == 2)
-        draw_from_segments<DT, 2>(P, row, n, P.parts, rec.M, zf, lim, Scale(P.T), sc);
+        draw_from_segments<DT, 2, kMassBits>(P, row, n, P.parts, rec.M, zf, lim, Scale(P.T), sc);
     else
-        draw_from_segments<DT, 1>(P, row, n, P.parts, rec.M, zf, lim, Scale(P.T), sc);
+        draw_from_segments<DT, 1, kMassBits>(P, row, n, P.parts, rec.M, zf, lim, Scale(P.T), sc);
 }
 
 template <int DT, bool VEC>

@@ -19,7 +19,7 @@ constexpr int NTF = 1024;              // threads per row workgroup
 constexpr int kWaves = NTF / kWave;    // 16
 constexpr int kIdBits = 18;            // ids < 2^18 in a support key
 constexpr int64_t kMaxV = 1 << kIdBits;
-constexpr double kFix = 1099511627776.0;  // 2^40: fixed-point unit of the masses
+constexpr int kMassBits = 40;  // the cuts' masses are in units of 2^-40
 
 // Largest k of the kernels that select from candidates in LDS (select.hip),
 // and the candidates they hold.
@@ -97,6 +97,8 @@ __device__ __forceinline__ float block_max_f(float v, float* s) {
     return t;
 }
 
+// exp(z - M) in units of 2^-BITS, rounded down.
+template <int BITS = kMassBits>
 __device__ __forceinline__ uint64_t weight_fx(float z, float M) {
     // NaN (and +inf against itself) carries no mass; -inf gives exp = 0.  No
     // branch, so that the chains of a thread's entries overlap.  The same
@@ -106,11 +108,20 @@ __device__ __forceinline__ uint64_t weight_fx(float z, float M) {
     const float e = exp_reduced(
         __builtin_amdgcn_fmed3f(d, -104.f, 0.f), [](float f) { return __builtin_amdgcn_exp2f(f); },
         [](float p, int n) { return __builtin_amdgcn_ldexpf(p, n); });
-    // floor(e * 2^40): both halves of the 24-bit product are exact.
-    const float f = d <= 0.f ? e * (float)kFix : 0.f;
+    const float f = d <= 0.f ? e * (float)(1ull << BITS) : 0.f;
+    // Both halves of the 24-bit product are exact.
     const uint32_t hi = (uint32_t)(f * 0x1p-32f);
     const uint32_t lo = (uint32_t)__builtin_fmaf((float)hi, -0x1p32f, f);
     return ((uint64_t)hi << 32) | lo;
+}
+
+// weight_fx for a draw, at least one unit where expf(z - M) is not 0: every kept
+// entry can be drawn.
+template <int BITS>
+__device__ __forceinline__ uint64_t draw_fx(float z, float M) {
+    const float d = z - M;
+    const uint64_t w = weight_fx<BITS>(z, M);
+    return d <= 0.f && d > -103.f && w == 0 ? 1 : w;
 }
 
 // Id of the q-th entry (1-based, ascending id) with key == v, by a pass in

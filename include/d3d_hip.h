@@ -411,8 +411,10 @@ size_t d3d_filter_rows_workspace_bytes(int N, int64_t V);
  * workgroup per row.  zfloor_out / zlimit_out [N] (both or neither), as
  * d3d_row_filter; tokens_out [N] (needs uniforms [N]) and probs_out [N] (may
  * be NULL): the inverse-CDF draw over the kept entries in id order and its
- * probability.  Masses are sums of exp(z - max z) in 2^-40 units.  Larger
- * top_k: D3D_E_UNSUPPORTED (d3d_row_filter takes any).
+ * probability.  The filter's masses are sums of exp(z - max z) in units of
+ * 2^-40, the draw's under a top-k of 2^-50 (2^-45 for rows with a long run of
+ * equal values at the cut).  Larger top_k: D3D_E_UNSUPPORTED (d3d_row_filter
+ * takes any).
  *
  * Replaces _sampling_probs' filters and _sample_with_prob,
  * single/eval_sync.py:287-338.
