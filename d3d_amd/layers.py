@@ -153,13 +153,16 @@ def rows64_silu_ok(H: int, K: int) -> bool:
 
 
 def rows_silu_ok(M: int, H: int, K: int) -> bool:
-    """rows64_silu_ok for M rows.  65-128 rows: grids of one round of tiles of
-    64 or 96 columns (12288 x 2048: 19.2 us against 19.1 and a SiLU-mul; 24576
-    x 4096: 50.6 against 52.9 and 5; its tiles of 128 are behind, 57).  129-192
-    rows: all (23.7 against 25.9, 60.9 against 60.4-64.9, before the SiLU-mul)."""
+    """rows64_silu_ok for M rows.  From 65 rows on a workgroup's products outlast
+    its share of the weights, so the tiles have to make about one round of the
+    256 CUs: 192 to 256 of 64 columns (12288 x 2048, 80 to 192 rows: 18.7-26.3 us
+    against 20.9-29.7 with the SiLU-mul; 8192 x 8192, 128 tiles: 55-76 against
+    42-68), or to 128 rows of 96 (24576 x 4096 in the target's forward, 4 layers,
+    80 / 96 / 128 rows: 836 / 869 / 927 us against 848 / 871 / 926; in tiles of 128
+    at 160 / 192 rows 1018 / 1086 against 1008 / 1081)."""
     if M > ROWS192 or not rows64_silu_ok(H, K):
         return False
-    return not ROWS64 < M <= 128 or H // 32 <= 256 or (H % 48 == 0 and H // 48 <= 256)
+    return M <= ROWS64 or 192 <= H // 32 <= 256 or (M <= 128 and H % 48 == 0 and 192 <= H // 48 <= 256)
 
 
 def gate_up_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

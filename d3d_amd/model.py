@@ -181,7 +181,7 @@ class Qwen3PagedModel(torch.nn.Module):
     def __init__(self, shape: ModelShape, device, *, draft: bool, seed: int = 0, init_std: float = 0.02):
         super().__init__()
         self.shape, self.draft, self.device = shape, draft, torch.device(device)
-        # Blocks of at most 64 tokens run their projections through
+        # Blocks of at most 192 tokens run their projections through
         # layers.project (the weight-streaming HIP GEMM where it is faster
         # than hipBLASLt) unless this is off.
         self.rows64_gemm = True
@@ -223,8 +223,7 @@ class Qwen3PagedModel(torch.nn.Module):
         weight-streaming HIP GEMM where layers.project / gate_up_silu pick it
         (when ``rows64_gemm``: the QKV, O and down GEMMs, whose K-split
         partials the next fused kernel sums, and the gate-up with the SiLU-mul
-        fused in, but for the target's at 65-128 rows); larger blocks use
-        F.linear.
+        fused in); larger blocks use F.linear.
         """
         B, Q = ids.shape
         s = self.shape
