@@ -2,9 +2,8 @@
 
 d3d_filter_rows must give the filter of d3d_row_filter (the general
 multi-pass selection) bit for bit: both place the cut with the same exact
-64-bit masses.  Its draw is checked against the draw of d3d_sample_rows under
-that filter, whose fp32 masses may cross a bar edge the other way.  Supports
-and top-k are checked against a stable CPU sort.
+64-bit masses.  Every row's draw must lie in its bar of the float64 CDF of the
+kept entries.  Supports and top-k are checked against a stable CPU sort.
 """
 from __future__ import annotations
 
@@ -53,17 +52,26 @@ def _general(x, T, k, p):
     return zf, lim
 
 
-def _draw(x, T, zf, lim, u):
-    N, V = x.shape
-    tok = torch.empty(N, dtype=torch.int64, device=DEV)
-    prob = torch.empty(N, device=DEV)
-    lib = _lib.load()
-    ws = torch.empty(lib.d3d_sample_workspace_bytes(N, V), dtype=torch.uint8, device=DEV)
-    st = lib.d3d_sample_rows(x.data_ptr(), _lib.dtype_code(x), N, V, T, None, zf.data_ptr(), lim.data_ptr(),
-                             u.data_ptr(), tok.data_ptr(), prob.data_ptr(), ws.data_ptr(), ws.numel(),
-                             _lib.stream_ptr(DEV))
-    _lib.check(st, "d3d_sample_rows")
-    return tok, prob
+def _check_draws(x, T, zf, lim, u, tok, prob):
+    """Each row's u lies in the drawn entry's bar of the fp64 CDF of the kept entries, ids in order."""
+    x, zf, lim, u, tok, prob = (t.cpu() for t in (x, zf, lim, u, tok, prob))
+    z = x.float() / torch.tensor(T)
+    ids = torch.arange(x.shape[1])
+    for n in range(x.shape[0]):
+        kept = (z[n] > zf[n]) | ((z[n] == zf[n]) & (ids <= lim[n]))
+        top = z[n][kept].max() if kept.any() else torch.tensor(-INF)
+        w = torch.where(kept, (z[n].double() - top.double()).exp(), 0.0).nan_to_num(0.0)
+        t = int(tok[n])
+        if not torch.isfinite(top):  # no entry has a weight
+            assert t == _lib.D3D_TOKEN_EMPTY_DISTRIBUTION and float(prob[n]) == 0
+            continue
+        q = w / w.sum()
+        hi = float(q[:t + 1].sum())
+        # z = x / T and z - max round to fp32: 2^-19 of a weight at |z| < 16; the
+        # masses' units are 2^-40 and finer
+        assert t >= 0 and bool(kept[t])
+        assert hi - float(q[t]) - 2e-6 <= float(u[n]) <= hi + 2e-6
+        assert abs(float(prob[n]) - float(q[t])) <= 4e-6 * float(q[t])
 
 
 @pytest.mark.parametrize("kind", ["plain", "ties", "flat", "masked", "odd", "sorted"])
@@ -82,19 +90,7 @@ def test_filter_rows_equals_the_general_filter(kind, V, k, p, dtype, T):
     torch.cuda.synchronize()
     assert torch.equal(got[0], zf) and torch.equal(got[1], lim)
     tok, prob = dr.sample_with_prob(x, T, k, p, uniforms=u)
-    rt, rp = _draw(x, T, zf, lim, u)
-    same = tok == rt
-    # The fp32 sums are good to ~1e-6 of the row's mass; only a draw that close
-    # to a bar edge (bars are ~1e-5 wide) may take the neighbour.
-    assert same.float().mean() >= 0.6
-    rows = torch.nonzero(same)[:, 0]
-    # blocked fp32 sums of positive terms: under 2^7 roundings of 2^-24 each side
-    assert torch.allclose(prob[rows], rp[rows], rtol=2e-5, atol=1e-9)
-    # The other rows drew a kept entry too.
-    for n in torch.nonzero(~same)[:, 0].tolist():
-        z = x[n].float() / T
-        t = int(tok[n])
-        assert t >= 0 and (z[t] > zf[n] or (z[t] == zf[n] and t <= lim[n]))
+    _check_draws(x, T, zf, lim, u, tok, prob)
 
 
 def test_filter_rows_takes_rows_in_batches():
@@ -115,30 +111,32 @@ def _sorted_ids(x, T, S):
     z = (x.float().cpu() / T).numpy().astype(np.float32)
     out = np.full((z.shape[0], S), -1, np.int64)
     for n, row in enumerate(z):
-        row = np.where(row == 0, np.float32(0), row)
-        key = np.where(np.isnan(row), -np.inf, row)
-        order = np.lexsort((np.arange(row.size), np.isnan(row), -key))
-        out[n] = order[:S]
+        ok = np.flatnonzero(~np.isnan(row))  # NaN entries are never selected
+        order = ok[np.lexsort((ok, -(row[ok] + np.float32(0))))][:S]
+        out[n, :order.size] = order
     return out
 
 
-@pytest.mark.parametrize("kind", ["plain", "ties", "flat", "masked", "sorted"])
+@pytest.mark.parametrize("kind", ["plain", "ties", "flat", "masked", "odd", "sorted"])
 @pytest.mark.parametrize("V,S", [(151936, 9), (151936, 64), (32771, 256), (32771, 512), (20000, 513), (9000, 4096),
                                  (16, 9), (12, 12)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_support_and_topk_match_a_stable_sort(kind, V, S, dtype):
-    N, T = 3, 0.8
+    N, T = 5 if kind == "odd" else 3, 0.8
     x = _rows(kind, N, V, dtype, V + S)
     u = torch.rand(N, generator=torch.Generator().manual_seed(S)).to(DEV)
     tok, ids, probs = dr.sample_with_sparse_probs(x, T, S, 0.95, uniforms=u)
     ref = _sorted_ids(x, T, S)
     np.testing.assert_array_equal(ids.cpu().numpy(), ref)
-    assert torch.allclose(probs.sum(-1), torch.ones(N, device=DEV), rtol=1e-5)
-    assert bool((ids == tok[:, None]).any(-1).all())
+    # Rows whose maximum is infinite (of either sign) have no distribution.
+    live = torch.isfinite(x.float().nan_to_num(-INF, INF, -INF).amax(-1) / T)
+    assert torch.allclose(probs.sum(-1), live.float(), rtol=1e-5)
+    assert torch.equal((ids == tok[:, None]).any(-1), live)
+    assert bool((tok[~live] == _lib.D3D_TOKEN_EMPTY_DISTRIBUTION).all())
     if S <= 64:
         top, vals = dr.topk_tokens(x, S, with_values=True)
         np.testing.assert_array_equal(top.cpu().numpy(), _sorted_ids(x, 1.0, S))
-        assert torch.equal(vals, x.float().gather(1, top))
+        assert torch.equal(vals, torch.where(top < 0, -INF, x.float().gather(1, top.clamp(min=0))))
 
 
 def test_masses_are_as_exact_as_the_exponential_allows():
