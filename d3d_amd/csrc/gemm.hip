@@ -22,8 +22,9 @@
 //   Other step counts of up to 64 rows run on gemm_rows64_dma_kernel (direct
 //   global -> LDS loads, two stages, two barriers per step).
 // * The tile per row count (us, graph-replayed on HBM-resident weights; the
-//   weights alone take 10.3 / 6.8 / 20.5 us at the copy rate for the target's
-//   qkv / o / down, 3.4 / 1.7 / 5.1 for the draft's):
+//   weights alone take 7.5 / 5.0 / 15.0 us for the target's qkv / o / down, 2.5
+//   / 1.3 / 3.8 for the draft's, at the 6.7 TB/s that a plain read of 4 GiB
+//   reaches -- a copy moves 4.9 and bounds no read):
 //     M <= 16, 32: four waves, TK 128.  In the 64-row kernel three quarters
 //       of the X loads, LDS traffic and MFMAs were repeats of the last row.
 //       16 rows: target 12.9 / 8.3 / 19.7 -> 11.5 / 7.5 / 18.7, draft
@@ -119,7 +120,7 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[4], uint16_t* y, f
 }
 
 // Direct global -> LDS form (global_load_lds, two stages): the kernel for
-// step counts gemm_rows64_kernel is not unrolled for.
+// step counts rows_kernel is not unrolled for.
 __global__ __launch_bounds__(NT) void gemm_rows64_dma_kernel(const uint16_t* __restrict__ x,
                                                          const uint16_t* __restrict__ w,
                                                          uint16_t* __restrict__ y, float* __restrict__ parts,

@@ -38,7 +38,7 @@ bool launch_steps(const SiluCall& c) {
 // Column tiles of 64 while they make at most one round of 256 workgroups, or
 // up to 32 rows, where a workgroup takes little of a CU; else of 96 where
 // those make a round, or of 128: fewer workgroups read X.  Target gate-up,
-// 24576 x 4096 (41.0 us at the copy rate), tiles of 64 / 96 / 128, us: 64 rows
+// 24576 x 4096 (30 us at the rate of a plain read), tiles of 64 / 96 / 128, us: 64 rows
 // 51.5 / 43.7 / 46.5 (hipBLASLt 49.5 and a SiLU-mul of 5), 128 rows 67.2 /
 // 50.6 / 57.0 (52.9), 192 rows 80.3 / 63.6 / 60.9 (60.4); 16 rows 43.1 with 64.
 int column_tile(int M, int H) {

@@ -61,18 +61,6 @@ __device__ __forceinline__ void for_row(const void* row, int V, float T, bool un
     for (int e = threadIdx.x; e < V; e += NTF) f(e, scaled<DT>(row, e, T, unit));
 }
 
-__device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t* s) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    __syncthreads();
-    if ((threadIdx.x & (kWave - 1)) == 0) s[threadIdx.x / kWave] = v;
-    __syncthreads();
-    uint32_t t = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) t += s[w];
-    return t;
-}
-
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* s) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);

@@ -98,7 +98,8 @@ def project(x: torch.Tensor, weight: torch.Tensor, max_rows: int = ROWS64) -> Pr
     """
     M, K = x.shape
     N = weight.shape[0]
-    if (M > min(max_rows, ROWS192) or weight.shape[1] != K or N % 64 or K % 128 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16
+    if (M > min(max_rows, ROWS192) or weight.shape[1] != K or N % 64 or K % 128
+            or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16
             or not x.is_contiguous() or not weight.is_contiguous()
             or x.data_ptr() % 16 or weight.data_ptr() % 16):  # the kernel's 16-byte row loads
         return F.linear(x, weight)

@@ -8,9 +8,10 @@ Reference behaviour (D3D repository):
 * single/eval_sync.py:713-717 and :763-768 -- the draft's argmax and
   ``torch.topk(log_softmax(logits), k)`` anchors.
 
-The kernel streams the weight once per 64 hidden rows, so it pays off up to
-64 rows (verify and recovery blocks of four requests); longer row sets are
-better served by a GEMM followed by ``draft.topk_tokens``.
+The kernel streams the weight once per 64 hidden rows, or per 128 above 64 rows
+at H of 2048 and 4096, so it pays off up to that many (verify and recovery
+blocks of four or eight requests); longer row sets are better served by a GEMM
+followed by ``draft.topk_tokens``.
 """
 from __future__ import annotations
 
@@ -19,7 +20,7 @@ import torch
 from . import _lib
 
 MAX_K = 8
-ROWS_PER_PASS = 64
+ROWS_PER_PASS = 64  # at every H; 128 above 64 rows at H of 2048 and 4096
 
 
 def lmhead_topk(hidden: torch.Tensor, weight: torch.Tensor, k: int, with_values: bool = False,
