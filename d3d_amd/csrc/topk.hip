@@ -51,8 +51,16 @@ constexpr int kMaxK = 64;
 constexpr int kBf16Chunks = 1;
 template <int DT>
 constexpr int chunks_per_wg() { return DT == kBF16 ? kBf16Chunks : 1; }
-// Largest k taken by rounds; wider ones (and V <= 2^18) go to select.hip.
-constexpr int rounds_max_k(int dtype) { return dtype == kF32 ? 4 : 8; }
+// Largest k taken by rounds; wider ones (and V <= 2^18) go to select.hip.  Many
+// rows of one or two chunks keep the rounds longer: their cost is k times a
+// few chunks, a selection's one 1,024-thread workgroup per row, 256 rows a
+// launch.  Rounds / selection, us: 4,096 rows of 1,000, bf16 k = 9 103 / 212, k
+// = 32 320 / 229, fp32 k = 9 125 / 198; 2,048 rows of 8,192, bf16 k = 9 65 / 127,
+// k = 32 193 / 129, fp32 k = 9 111 / 124; 1,088 rows of 32,000, bf16 k = 9 78 / 62.
+inline int rounds_max_k(int dtype, int N, int64_t V) {
+    if (N > 256 && V <= 2 * kChunk) return dtype == kF32 ? (V <= kChunk ? 14 : 10) : 18;
+    return dtype == kF32 ? 4 : 8;
+}
 constexpr int kMaxCand = 8192;  // chunk candidates per row merged in LDS
 
 struct Cand {
@@ -687,15 +695,17 @@ static size_t cand_bytes(int N, int64_t V, int k) {
     return ((size_t)N * C * k * sizeof(topk::Cand) + 255) & ~(size_t)255;
 }
 
-static bool topk_selects(int dtype, int64_t V, int k) { return k > topk::rounds_max_k(dtype) && V <= filt::kMaxV; }
+static bool topk_selects(int dtype, int N, int64_t V, int k) {
+    return k > topk::rounds_max_k(dtype, N, V) && V <= filt::kMaxV;
+}
 
 extern "C" size_t d3d_topk_workspace_bytes(int N, int64_t V, int k) {
     if (N < 1 || V < 1 || k < 1) return 0;
     const size_t C = (size_t)((V + rows::kChunk - 1) / rows::kChunk);
     // The dtype is not known here: room for whichever way it takes.
     size_t bytes = 0;
-    if (topk_selects(D3D_DTYPE_F32, V, k)) bytes = filt::select_scratch_bytes(N, (int)C, true);
-    if (!topk_selects(D3D_DTYPE_BF16, V, k))
+    if (topk_selects(D3D_DTYPE_F32, N, V, k)) bytes = filt::select_scratch_bytes(N, (int)C, true);
+    if (!topk_selects(D3D_DTYPE_BF16, N, V, k))
         bytes = std::max(bytes, cand_bytes(N, V, k) + (((size_t)N * C * sizeof(float2) + 255) & ~(size_t)255));
     return bytes;
 }
@@ -718,7 +728,7 @@ extern "C" int d3d_topk_rows(const void* logits, int dtype, int N, int64_t V, in
     P.k = k;
     if ((int64_t)P.C * k > kMaxCand) return D3D_E_SHAPE;
     if (workspace_bytes < d3d_topk_workspace_bytes(N, V, k)) return D3D_E_WORKSPACE;
-    if (topk_selects(dtype, V, k))
+    if (topk_selects(dtype, N, V, k))
         return (int)filt::select_topk(logits, dtype, N, (int)V, k, log_softmax && vals_out, ids_out, vals_out,
                                       workspace, static_cast<hipStream_t>(stream));
     P.cand = static_cast<Cand*>(workspace);

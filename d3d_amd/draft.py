@@ -124,11 +124,22 @@ def _filter_args(V: int, top_k: int, top_p: Optional[float]) -> Tuple[int, float
     return k, p, (k > 0 or p < 1.0) and k <= _lib.FILTER_MAX_K and V <= _lib.FILTER_MAX_V
 
 
+def _rounds_max_k(logits: torch.Tensor) -> int:
+    """The k up to which many short rows [N, V] do better with d3d_topk_rows'
+    rounds than with a selection by one workgroup per row (else 0).  4,096 bf16
+    rows of 1,000, draw under a top-5: 127 us against 287."""
+    V = logits.shape[-1]
+    if logits.numel() // V <= 256 or V > 8192:
+        return 0
+    return 18 if logits.dtype == torch.bfloat16 else (14 if V <= 4096 else 10)
+
+
 def _top_k_floor(logits: torch.Tensor, k: int, p: float, fused: bool) -> Optional[torch.Tensor]:
     """The k-th largest logit of each row [N, V] for a top-k filter alone that
     the top-k kernels take and d3d_filter_rows does not, else None.  That is
-    rows past 2^18 entries: 64 rows of 300,000, k = 5 a draw of 54 us against
-    590 with d3d_row_filter, k = 50 302 against 597."""
+    many short rows (_rounds_max_k) and rows past 2^18 entries: 64 rows of
+    300,000, k = 5 a draw of 54 us against 590 with d3d_row_filter, k = 50 302
+    against 597."""
     V = logits.shape[-1]
     if fused or p < 1.0 or not 0 < k <= _lib.TOPK_MAX_K or -(-V // 4096) * k > _lib.TOPK_MAX_CANDIDATES:
         return None
@@ -179,6 +190,7 @@ def sample_with_prob(logits: torch.Tensor, temperature: float = 0.0, top_k: int 
     greedy = not temperature > 1e-5
     u = None if greedy else _uniforms(lg.shape[:-1], dev, uniforms, generator)
     k, p, fused = (0, 1.0, False) if greedy else _filter_args(V, top_k, top_p)
+    fused = fused and (p < 1.0 or k > _rounds_max_k(lg))
     tok = torch.empty(lg.shape[:-1], dtype=torch.int64, device=dev)
     prob = torch.empty(lg.shape[:-1], dtype=torch.float32, device=dev)
     lib = _lib.load()
@@ -222,6 +234,7 @@ def sampling_probs(logits: torch.Tensor, temperature: float = 0.0, top_k: int = 
     N = lg.numel() // V
     greedy = not temperature > 1e-5
     k, p, fused = (0, 1.0, False) if greedy else _filter_args(V, top_k, top_p)
+    fused = fused and (p < 1.0 or k > _rounds_max_k(lg))
     kth = _top_k_floor(lg, k, p, fused)
     zf, lim = (None, None) if kth is not None else _filters(lg, temperature, k, p, fused)
     out = torch.empty(lg.shape, dtype=torch.float32, device=dev)
@@ -244,9 +257,9 @@ def sample_with_sparse_probs(logits: torch.Tensor, temperature: float, top_k: in
     probabilities are softmax(z) over the support after the nucleus filter
     (``top_p`` < 1: entry s > 0 is dropped when the mass of entries 0..s-1
     exceeds top_p), and the token is the inverse-CDF draw from them in
-    support order.  Supports of up to 8 entries, and up to 64 of rows the
-    sorted-support path does not take (V > 2^18), take the top-k kernels and one
-    wave per row; the others the sorted-support path.
+    support order.  Supports of up to 8 entries (32 above 256 rows), and up to
+    64 of rows the sorted-support path does not take (V > 2^18), take the top-k
+    kernels and one wave per row; the others the sorted-support path.
     """
     dev = _lib.require_device(logits)
     if not temperature > 1e-5:
@@ -264,7 +277,10 @@ def sample_with_sparse_probs(logits: torch.Tensor, temperature: float, top_k: in
     u = _uniforms(lg.shape[:-1], dev, uniforms, generator)
     tok = torch.empty(lg.shape[:-1], dtype=torch.int64, device=dev)
     probs = torch.empty(*lg.shape[:-1], S, dtype=torch.float32, device=dev)
-    if S > 64 or (S > 8 and V <= _lib.FILTER_MAX_V):
+    # Above 256 rows a wave per row draws what 1,024 threads do more slowly
+    # (1,088 bf16 rows of 32,000, S = 9: 67 us against 94).
+    few = 32 if N > 256 else 8
+    if S > 64 or (S > few and V <= _lib.FILTER_MAX_V):
         ids = torch.empty(*lg.shape[:-1], S, dtype=torch.int64, device=dev)
         lib = _lib.load()
         nbytes = lib.d3d_support_workspace_bytes(max(N, 1), S)
