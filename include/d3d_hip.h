@@ -438,7 +438,9 @@ size_t d3d_support_workspace_bytes(int N, int S);
  * probability.  T > 1e-5, 0 < top_p <= 1.  Workspace:
  * d3d_support_workspace_bytes(N, S).  Two launches for S <= 4096 (a
  * selection in LDS), a segmented sort above.  d3d_topk_rows +
- * d3d_sample_support cover S <= 64 too and are faster up to 8.
+ * d3d_sample_support cover S <= 64 too and are faster up to 8, and above 256
+ * rows up to 32.  A row with fewer than S entries that are not NaN ends in id
+ * -1 (S <= 64 or S = V) or in its first NaN ids, with probability 0.
  */
 int d3d_sample_support_wide(const void* logits, int dtype, int N, int64_t V, float temperature, int S,
                             float top_p, const float* uniforms, int64_t* tokens_out, int64_t* support_ids_out,
